@@ -989,6 +989,10 @@ struct Group {
                 return false;
             }
         }
+        uint64_t freed[kW];
+#pragma unroll
+        for (int w = 0; w < kW; ++w) freed[w] = rem[w] & ~added[w];
+        retire_vertices(freed);
 #pragma unroll
         for (int w = 0; w < kW; ++w) valid[w] = (valid[w] & ~rem[w]) | added[w];
         dirty = true;
@@ -1048,6 +1052,36 @@ struct Group {
         return !too_far(c);
     }
 
+    // May the plane of the lane's own candidate cut the cell: is some vertex
+    // not certainly behind it (the test of beyond32, so a candidate refused
+    // here would be refused vertex by vertex in clip())?  The slots are read
+    // in order, each by the whole group at once; a free slot holds a radius
+    // that fails the test (retire_vertices).
+    __device__ __forceinline__ bool may_cut(const Cand &c) const {
+        const float c2 = fmaf(kG32, c.pH, kTiny32);
+        bool hit = false;
+#pragma unroll 1
+        for (int v = 0; v < V; v += 8) {
+            if (__ballot((valid[v >> 6] >> (v & 63)) != 0ull) == 0ull) break;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const float4 p = S->vpos[v + u];
+                const float Pv = fmaf(c.ax, p.x, fmaf(c.ay, p.y, fmaf(c.az, p.z, -c.H)));
+                hit |= !(Pv < -fmaf(c.pa1, p.w, c2));
+            }
+        }
+        return hit;
+    }
+
+    // Marks the slots of m as free for may_cut().
+    __device__ __forceinline__ void retire_vertices(const uint64_t (&m)[kW]) const {
+        if constexpr (G == 16) {
+#pragma unroll
+            for (int k = 0; k < kRows; ++k)
+                if (own(m, k)) S->vpos[gl + G * k] = make_float4(0.f, 0.f, 0.f, -FLT_MAX);
+        }
+    }
+
     // Offers a batch of up to G candidates (lane-specific j when `has`).
     __device__ __forceinline__ void offer_batch(bool has, uint32_t j) {
         Cand c;
@@ -1063,6 +1097,16 @@ struct Group {
         if (gl == 0 && skipped) count(kStatSkipped, (uint32_t)__popcll(skipped));
         uint64_t todo = gballot(live_c);
         if (gl == 0 && todo) count(kStatCandidates, (uint32_t)__popcll(todo));
+        if constexpr (G == 16) {
+            // Every vertex against the lane's own candidate: one that lies
+            // certainly behind all of them does not cut (the cell only shrinks
+            // after this), so only the others are offered one at a time.
+            // Nothing to gain on the initial box, which every guess cuts.
+            if (np > 6 && todo) {
+                todo = gballot(live_c && may_cut(c));
+                if (!todo) return;
+            }
+        }
         if (live_c) {
             C->aH[gl] = make_float4(c.ax, c.ay, c.az, c.H);
             // the owner's sign bit marks a candidate that may already own a plane
@@ -1137,8 +1181,13 @@ struct Group {
             if (sgn > 0) make_vertex(gl, X, Y, Z);
             else make_vertex(gl, X, Z, Y);
         }
+        uint64_t unused[kW];
 #pragma unroll
-        for (int w = 0; w < kW; ++w) valid[w] = w == 0 ? 0xFFull : 0ull;
+        for (int w = 0; w < kW; ++w) {
+            valid[w] = w == 0 ? 0xFFull : 0ull;
+            unused[w] = ~valid[w];
+        }
+        retire_vertices(unused);
         bloom = 0;
         update_bounds();
         dirty = false;
