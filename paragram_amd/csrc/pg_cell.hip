@@ -27,6 +27,7 @@
 #include "pg_common.hpp"
 #include "pg_exact.hpp"
 #include "pg_kernels.hpp"
+#include "pg_wide.hpp"
 
 #include <float.h>
 
@@ -45,6 +46,7 @@ struct CellParams {
     const uint32_t *perm;   // sorted -> original
     const uint32_t *inv;    // original -> sorted
     const Node *nodes;
+    const WideChild *wide;  // the 16-wide form, 16 per record
     const uint32_t *dup_head;
     const uint32_t *dup_next;
     int64_t begin, end;
@@ -111,6 +113,7 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
 }  // namespace pg
 
 #include "pg_group_cell.hpp"
+#include "pg_tier0_cell.hpp"
 
 namespace pg {
 
@@ -189,6 +192,7 @@ hipError_t launch_cells(const CellArgs &a, hipStream_t stream) {
     prm.perm = (const uint32_t *)(ws + L.perm);
     prm.inv = (const uint32_t *)(ws + L.inv);
     prm.nodes = (const Node *)(ws + L.nodes);
+    prm.wide = (const WideChild *)(ws + L.boxes);
     prm.dup_head = (const uint32_t *)(ws + L.dup_head);
     prm.dup_next = (const uint32_t *)(ws + L.dup_next);
     prm.begin = a.begin;

@@ -128,7 +128,7 @@ struct IndexLayout {
     uint64_t children;   // uint32 [2*(n-1)]  Karras child codes
     uint64_t parents;    // uint32 [2n-1]     parent of internal (0..n-2) and leaf (n-1..2n-2)
     uint64_t ranges;     // uint2  [n-1]      covered range of internal nodes
-    uint64_t boxes;      // float4 [2*(n-1)]  internal node AABB lo/w, hi
+    uint64_t boxes;      // float4 [2*(n-1)]  internal node AABB lo/w, hi (after the build: the wide form)
     uint64_t flags;      // uint32 [n-1]      refit arrival counters
     uint64_t reduce;     // float  [6 * reduce_blocks]
     uint64_t scan_tmp;   // uint32 block sums of the histogram scan

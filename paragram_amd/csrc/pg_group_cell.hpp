@@ -1,10 +1,12 @@
-// Cooperative cell construction: G lanes build one cell together, with the
-// whole cell in LDS.  Included by pg_cell.hip (it uses CellParams, the
-// precision constants and the plane-triple helpers defined there).
+// The FP64-capable tiers: G lanes build one cell together, with the whole
+// cell in LDS.  Included by pg_cell.hip (it uses CellParams, the precision
+// constants and the plane-triple helpers defined there), before
+// pg_tier0_cell.hpp, the FP32-only tier that every cell starts in.
 //
-// Four instances (capacity tiers):
-//   tier 0: G = 16 lanes, 64 vertex slots, 48 plane slots (about 3.3 KB of
-//           LDS per cell, 4 cells per wave) -- every cell starts here;
+// Four instances:
+//   tier 0's twin: G = 16 lanes, 64 vertex slots, 48 plane slots (about
+//           3.3 KB of LDS per cell, 4 cells per wave) -- the cells tier 0
+//           gave up on for their precision;
 //   tier m: G = 64 lanes, 192 vertex slots, 128 plane slots (one cell per
 //           wave, 12 waves per CU) -- the few cells that outgrow tier 0
 //           (cells with more than about 34 faces);
@@ -23,9 +25,8 @@
 //   plx[P]   float2  permanent of H and the owner (sorted point id, or a
 //                    negative box-plane code)
 //   tmp[V]   uint32  clip and emission scratch
-//   pm[P/2]  uint32  (tier 0) per plane, a 16-bit mask of the lanes whose
+//   pm[P/2]  uint32  (16 lanes) per plane, a 16-bit mask of the lanes whose
 //                    removed triangle holds the plane; zero between clips
-//   tent[8]  2 x u32 (tier 0) removal tests taken by their FP32 sign
 // Vertices live in a pool of V slots with a group-uniform valid mask (slot
 // v = lane + G k belongs to lane v mod G), so a clip frees and refills slots
 // without moving data.
@@ -34,7 +35,7 @@
 // (one per lane, then offered in order), the boundary edges of a clip and
 // the new vertices they make, bounds reductions and the row sort.  All
 // control decisions are group-uniform (ballots restricted to the group).
-// The cells of one wave (Morton neighbours) share one best-first traversal.
+// The cells of one wave (Morton neighbours) share one depth-first traversal.
 #pragma once
 
 namespace pg {
@@ -49,13 +50,6 @@ struct alignas(16) GroupLDS {
     uint32_t pm[P <= 64 ? (P + 1) / 2 : 1];
     uint32_t ctr[kNumCtr];  // diagnostics, in the order of the statistics slots
     uint32_t exact_events;  // removal tests of the current cell decided by expansion arithmetic
-    // (tier 0) removal tests taken by their FP32 sign: the vertex's plane
-    // triple (slots, kept and renumbered by the plane collection), and the
-    // query point with the sign taken in bit 31
-    uint32_t tent[P <= 64 ? kTentMax : 1][2];
-    // their number (every lane of the group writes it, with the same value,
-    // so each lane reads back its own store)
-    uint32_t ntent;
 };
 
 // Candidates of one batch, staged for the group: (a, H) and (pH, owner).
@@ -385,10 +379,7 @@ __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirs
 __device__ __forceinline__ float uniform(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
 
 // ------------------------------------------------------------------ group
-// kExact: the tier carries the FP64 recheck path.  A tier without it gives
-// up on a cell at the first test its FP32 filter cannot decide (`bail`), and
-// the cell is rebuilt by the FP64-capable twin of the tier.
-template <int G, int V, int P, int L, bool kExact>
+template <int G, int V, int P, int L>
 struct Group {
     static constexpr int kRows = V / G;               // vertex slots per lane
     static constexpr int kW = V / 64;                 // words of a vertex mask
@@ -399,7 +390,6 @@ struct Group {
     static constexpr uint32_t kBMask = (1u << kB) - 1u;
     static_assert((G == 16 || G == 64) && L % kWave == 0 && V % 64 == 0 && P < (1 << kB) && 3 * kRows <= 64, "group geometry");
 
-    static constexpr bool kIsExact = kExact;
     static constexpr int kLS = L / kWave;  // wait-list slots per lane
     GroupLDS<V, P> *S;
     CandLDS<G> *C;
@@ -424,12 +414,7 @@ struct Group {
     float EM_;           // largest vertex error radius w of the cell
     bool bounded;
     int status;
-    bool overflow;  // the cell left this tier (capacity, or `bail`)
-    // why an FP32-only tier gave the cell up (0: it did not): 1 an undecided
-    // removal test, 2 an undecided vertex orientation, 3 a predicted cube
-    // that cut the cell (counted per cell after the traversal)
-    uint32_t bail;
-    bool cube;      // the cell started inside a predicted cube (see init_box)
+    bool overflow;  // the cell left this tier (capacity)
     bool active;  // the group holds a cell in this round
     bool dirty;   // the cell changed since the AABB was computed
     uint64_t bloom;
@@ -510,13 +495,11 @@ struct Group {
     // |N - N~| <= g pN and |D - D~| <= g pD (g = 2e-6), the position error is
     // |y - N~/D~| <= (g pN + |y~| g pD) / (D~ - g pD), plus division rounding.
     // Returns false when the FP32 orientation is not safely positive: the
-    // slot then holds radius -1 and fix_vertices() replaces it.  The tiers
-    // with an FP64 path also leave to it the ill-conditioned vertices, whose
-    // FP32 radius exceeds 2^-12 of the position (nearly parallel or coaxial
-    // planes): one such vertex in a cell inflates its bounds until no node or
-    // candidate can be pruned and every test needs FP64.  (The FP32-only
-    // tier keeps them: an FP64 call site there costs it registers on every
-    // cell, and a test such a vertex leaves open sends the cell to the twin.)
+    // slot then holds radius -1 and fix_vertices() replaces it, as it does the
+    // ill-conditioned vertices, whose FP32 radius exceeds 2^-12 of the position
+    // (nearly parallel or coaxial planes): one such vertex in a cell inflates
+    // its bounds until no node or candidate can be pruned and every test needs
+    // FP64.
     __device__ __forceinline__ bool make_vertex(int slot, uint32_t i, uint32_t j, uint32_t k) {
         const float4 A = S->pl[i], B = S->pl[j], C = S->pl[k];
         const float pHA = S->plx[i].x, pHB = S->plx[j].x, pHC = S->plx[k].x;
@@ -551,13 +534,11 @@ struct Group {
             const float ey = (kG32 * pNy + fabsf(y) * eD) * den + fabsf(y) * kSlack;
             const float ez = (kG32 * pNz + fabsf(z) * eD) * den + fabsf(z) * kSlack;
             pos = make_float4(x, y, z, fmaxf(ex, fmaxf(ey, ez)) + kTiny32);
-            if constexpr (kExact) {
-                if (pos.w > 0x1p-12f * fmaxf(fabsf(x), fmaxf(fabsf(y), fabsf(z)))) {
-                    pos.w = -1.0f;
-                    ok = false;
-                }
+            if (pos.w > 0x1p-12f * fmaxf(fabsf(x), fmaxf(fabsf(y), fabsf(z)))) {
+                pos.w = -1.0f;
+                ok = false;
             }
-        } else if (D < -eD && pD > kTiny32 && (kExact || S->ntent == 0u)) {
+        } else if (D < -eD && pD > kTiny32) {
             count(kStatInconsistent);
         }
         store_vertex(slot, pos);
@@ -592,8 +573,7 @@ struct Group {
 
     // Is vertex v strictly beyond the plane of q?  Filter: the error of
     // a~ . y~ - H~ against a . y - H is at most |a|_1 eps + 2e-6 (sum |a_k y_k| + pH).
-    // Returns 1 (beyond), 0 (not beyond), or when undecided (FP64 recheck)
-    // -2 if the FP32 value is positive and -1 if not.
+    // Returns 1 (beyond), 0 (not beyond) or -1 (undecided: FP64 recheck).
     // (with the stored w: |a|_1 w + 2e-6 pH + tiny bounds the error of the
     // FMA chain below against a . y - H)
     __device__ __forceinline__ int beyond32(int v, const Cand &q) const {
@@ -601,7 +581,7 @@ struct Group {
         const float Pv = fmaf(q.ax, p.x, fmaf(q.ay, p.y, fmaf(q.az, p.z, -q.H)));
         const float err = fmaf(q.pa1, p.w, q.c2);
         if (fabsf(Pv) > err) return Pv > 0.0f ? 1 : 0;
-        return Pv > 0.0f ? -2 : -1;
+        return -1;
     }
 
     // ---------------------------------------------------------- bounds
@@ -749,24 +729,10 @@ struct Group {
         return (uint32_t)r;
     }
 
-    // Drops unreferenced planes and renumbers the vertex triples (the planes
-    // of a recorded test's vertex stay, renumbered too, until the record is
-    // written out with the cell).
+    // Drops unreferenced planes and renumbers the vertex triples.
     __device__ __forceinline__ void garbage_collect() {
         uint64_t used[kPW];
         used_planes(used);
-        const uint32_t nt = kExact ? 0u : S->ntent;
-        if constexpr (!kExact) {
-            for (uint32_t i = 0; i < nt; ++i) {
-                const uint32_t t = S->tent[i][0];
-#pragma unroll
-                for (int e = 0; e < 3; ++e) {
-                    const uint32_t p = tri_get<kB>(t, e);
-#pragma unroll
-                    for (int w = 0; w < kPW; ++w) used[w] |= (int)(p >> 6) == w ? (1ull << (p & 63)) : 0ull;
-                }
-            }
-        }
 #pragma unroll
         for (int k = 0; k < kPRows; ++k) {
             const int p = gl + G * k;
@@ -794,13 +760,6 @@ struct Group {
                                          plane_rank(used, tri_get<kB>(t, 2)));
             }
         }
-        if constexpr (!kExact) {
-            if ((uint32_t)gl < nt) {
-                const uint32_t t = S->tent[gl][0];
-                S->tent[gl][0] = tri_pack<kB>(plane_rank(used, tri_get<kB>(t, 0)),
-                                              plane_rank(used, tri_get<kB>(t, 1)), plane_rank(used, tri_get<kB>(t, 2)));
-            }
-        }
         np = mask_popc(used);
     }
 
@@ -821,43 +780,18 @@ struct Group {
         uint64_t rem[kW];
 #pragma unroll
         for (int w = 0; w < kW; ++w) rem[w] = 0;
-        uint32_t mine = 0, unsure = 0, lean = 0;
+        uint32_t mine = 0, unsure = 0;
 #pragma unroll
         for (int k = 0; k < kRows; ++k) {
             if (!own(valid, k)) continue;
             const int b = beyond32(gl + G * k, q);
             if (b > 0) mine |= 1u << k;
             if (b < 0) unsure |= 1u << k;
-            if (b == -2) lean |= 1u << k;
         }
-        if constexpr (kExact) {
-            while (unsure) {  // one FP64 call site
-                const int k = (int)__builtin_ctz(unsure);
-                unsure &= unsure - 1u;
-                if (recheck64(gl + G * k, q.owner)) mine |= 1u << k;
-            }
-        } else if (gany(unsure != 0u)) {
-            // Undecided in FP32: take the sign of the FP32 value and record
-            // the test; a pass after this tier decides it in FP64 and sends
-            // the cell to the FP64-capable twin if the sign was wrong.  A
-            // cell with more such tests than its record holds goes there now.
-            const uint32_t n0 = S->ntent;
-            int tot;
-            uint32_t r = n0 + (uint32_t)gexcl(__popc(unsure), tot);
-            if (n0 + (uint32_t)tot > (uint32_t)kTentMax) {
-                overflow = true;
-                bail = 1u;
-                return false;
-            }
-            while (unsure) {
-                const int k = (int)__builtin_ctz(unsure);
-                unsure &= unsure - 1u;
-                S->tent[r][0] = S->vtri[gl + G * k];
-                S->tent[r][1] = (uint32_t)q.owner | (((lean >> k) & 1u) << 31);
-                ++r;
-            }
-            S->ntent = n0 + (uint32_t)tot;
-            mine |= lean;
+        while (unsure) {  // one FP64 call site
+            const int k = (int)__builtin_ctz(unsure);
+            unsure &= unsure - 1u;
+            if (recheck64(gl + G * k, q.owner)) mine |= 1u << k;
         }
         if (!gany(mine != 0u)) return false;  // no vertex beyond: the plane does not cut
 #pragma unroll
@@ -951,8 +885,7 @@ struct Group {
         // every plane of the boundary cycle starts one edge and ends one
         if (nb < 3 || gsum(sx_) != gsum(sy_)) {
             status = kInconsistentBoundary;
-            // (after a test taken by its FP32 sign the cell is rebuilt instead)
-            if (gl == 0 && (kExact || S->ntent == 0u)) count(kStatInconsistent);
+            if (gl == 0) count(kStatInconsistent);
             return true;
         }
         uint64_t freem[kW];
@@ -980,15 +913,7 @@ struct Group {
         }
         uint64_t added[kW];
         mask_first(freem, nb, added);
-        if (gany(bad)) {
-            if constexpr (kExact) {
-                fix_vertices(added);
-            } else {
-                overflow = true;
-                bail = 2u;
-                return false;
-            }
-        }
+        if (gany(bad)) fix_vertices(added);
         uint64_t freed[kW];
 #pragma unroll
         for (int w = 0; w < kW; ++w) freed[w] = rem[w] & ~added[w];
@@ -1147,30 +1072,23 @@ struct Group {
         }
     }
 
-    // The initial cell: the box, or (cube_h > 0, a predicted half-width in
-    // doubled coordinates) the box cut by the cube |y_k| <= cube_h, whose
-    // planes carry owner codes -7..-12.  A cell whose final vertices touch a
-    // cube plane, or that empties, is rebuilt without the cube.
-    __device__ __forceinline__ void init_box(float cube_h = 0.0f) {
-        bool from_cube = false;
+    // The initial cell: the box.
+    __device__ __forceinline__ void init_box() {
         if (gl < 6) {
             const int axis = gl >> 1, side = gl & 1;
             // (a lane-dependent choice among the members sx, sy, sz would be
             // compiled into a choice of addresses, moving them to scratch)
             const float4 sp = pts[seed];
             const float s = axis == 0 ? sp.x : (axis == 1 ? sp.y : sp.z);
-            float h = side ? 2.0f * (hdr->box_hi[axis] - s) : 2.0f * (s - hdr->box_lo[axis]);
-            from_cube = cube_h > 0.0f && cube_h < h;
-            if (from_cube) h = cube_h;
+            const float h = side ? 2.0f * (hdr->box_hi[axis] - s) : 2.0f * (s - hdr->box_lo[axis]);
             float4 pl = make_float4(0.f, 0.f, 0.f, h);
             const float sg = side ? 1.0f : -1.0f;
             if (axis == 0) pl.x = sg;
             if (axis == 1) pl.y = sg;
             if (axis == 2) pl.z = sg;
             S->pl[gl] = pl;
-            S->plx[gl] = make_float2(fabsf(h), __int_as_float((from_cube ? -7 : -1) - gl));
+            S->plx[gl] = make_float2(fabsf(h), __int_as_float(-1 - gl));
         }
-        cube = gany(from_cube);
         np = 6;
         // the 8 corners go to slots 0..7 (lanes 0..7 of row 0)
         if (gl < 8) {
@@ -1413,33 +1331,15 @@ struct Group {
         }
     }
 
-    // Does a final vertex lie on a plane of the predicted cube (group op)?
-    __device__ __forceinline__ bool cube_touched() const {
-        uint64_t used[kPW];
-        used_planes(used);
-        bool hit = false;
-#pragma unroll
-        for (int k = 0; k < kPRows; ++k) {
-            const int p = gl + G * k;
-            if (p < np && mask_bit(used, p)) hit |= __float_as_int(S->plx[p].y) <= -7;
-        }
-        return gany(hit);
-    }
-
     __device__ __forceinline__ void start(uint32_t cell, const CellParams &prm) {
         seed = cell;
-        if constexpr (kExact) {
-            if (gl == 0) S->exact_events = 0u;
-        } else {
-            S->ntent = 0u;
-        }
+        if (gl == 0) S->exact_events = 0u;
         const float4 s = pts[cell];
         sx = s.x, sy = s.y, sz = s.z, sw = s.w;
         status = kSuccess;
         overflow = false;
-        bail = 0u;
         const uint32_t orig = perm[cell];
-        init_box((!kExact && prm.init_h) ? 2.0f * prm.init_h[orig] : 0.0f);
+        init_box();
         in_guess = true;
         bloom_all = false;
         guess_r2 = 0.0f;
@@ -1565,19 +1465,11 @@ constexpr int kT0Lanes = 16, kT0Verts = 64, kT0Planes = 48, kT0List = 128, kT0Th
 constexpr int kTmLanes = 64, kTmVerts = 192, kTmPlanes = 128, kTmList = 128, kTmThreads = 128;
 constexpr int kT1Lanes = 64, kT1Verts = 512, kT1Planes = 255, kT1List = 128, kT1Threads = 128;
 constexpr int kT2Lanes = 64, kT2Verts = 1024, kT2Planes = 1023, kT2List = 128, kT2Threads = 64;
-using Tier0 = Group<kT0Lanes, kT0Verts, kT0Planes, kT0List, false>;
-using Tier0x = Group<kT0Lanes, kT0Verts, kT0Planes, kT0List, true>;
-using TierM = Group<kTmLanes, kTmVerts, kTmPlanes, kTmList, true>;
-using Tier1 = Group<kT1Lanes, kT1Verts, kT1Planes, kT1List, true>;
-using Tier2 = Group<kT2Lanes, kT2Verts, kT2Planes, kT2List, true>;
+using Tier0x = Group<kT0Lanes, kT0Verts, kT0Planes, kT0List>;
+using TierM = Group<kTmLanes, kTmVerts, kTmPlanes, kTmList>;
+using Tier1 = Group<kT1Lanes, kT1Verts, kT1Planes, kT1List>;
+using Tier2 = Group<kT2Lanes, kT2Verts, kT2Planes, kT2List>;
 
-// Tier 0: a wave holds four cells per round and traverses for them
-// together.  The FP32-only instance takes Morton-consecutive cells of the
-// range from a global counter; a cell it gives up on (`bail`) is flagged for
-// the FP64-capable instance (kExact), whose waves scan the flags in windows
-// of 64 Morton-consecutive cells and take the flagged cells four at a time
-// (neighbours again, so the shared traversal stays coherent).  A cell that
-// outgrows the tier is queued for tier m.
 // The address of the block's copy of the launch's parameters (in LDS: one
 // copy per block, where a kernel argument whose address is taken would be
 // copied per lane to scratch), opaque to the optimiser: fields read through
@@ -1618,11 +1510,12 @@ __device__ __forceinline__ uint64_t pool_take(const CellParams &P, uint32_t n) {
     return ((uint64_t)rl((uint32_t)(b >> 32), 0) << 32) | (uint64_t)rl((uint32_t)b, 0);
 }
 
-// kFlagged: the instance that takes the cells flagged by the first one
-// (else the cells of the range, or the batch's quads).
-template <typename T, bool kFlagged>
-__device__ __forceinline__ void tier0_body(const CellParams &prm) {
-    constexpr bool kExactTier = kFlagged;
+// Tier 0's twin: the waves scan the flags of the range in windows of 64
+// Morton-consecutive cells and take the flagged cells four at a time
+// (neighbours, so the shared traversal stays coherent).  A cell that outgrows
+// it is queued for tier m.
+template <typename T>
+__device__ __forceinline__ void tier0x_body(const CellParams &prm) {
     constexpr int kCellsPerWave = kWave / kT0Lanes;
     __shared__ GroupLDS<kT0Verts, kT0Planes> lds[kT0Threads / kT0Lanes];
     __shared__ CandLDS<kT0Lanes> cands[kT0Threads / kT0Lanes];
@@ -1638,8 +1531,8 @@ __device__ __forceinline__ void tier0_body(const CellParams &prm) {
     __syncthreads();
     const int lane = threadIdx.x & (kWave - 1);
     const int grp = lane / kT0Lanes;
-    if (kExactTier && prm.counters[5] == 0u) return;  // no cell was flagged
-    if (kExactTier && prm.counters[5] <= kFewFlagged) {
+    if (prm.counters[5] == 0u) return;  // no cell was flagged
+    if (prm.counters[5] <= kFewFlagged) {
         // a few flagged cells: queued for tier m, with no plane owners (the
         // flags read in a grid-stride loop: no work counter to contend for)
         const int64_t count = prm.end - prm.begin;
@@ -1671,38 +1564,7 @@ __device__ __forceinline__ void tier0_body(const CellParams &prm) {
         // rather than kept in registers across the traversal
         const CellParams &P = *reread(&sprm);
         const uint32_t orig = P.perm[cell];
-        if (kExactTier && active && g.gl == 0 && g.S->exact_events) log_exact(P, orig, g.S->exact_events);
-        // a cell built inside a predicted cube stands only if the cube cut nothing
-        if (active && !kExactTier && !g.overflow && g.cube && (g.status != kSuccess || g.cube_touched()))
-            g.overflow = true, g.bail = 3u;
-        if constexpr (!kExactTier) {
-            // the removal tests taken by their FP32 sign go to the record for
-            // the FP64 check after this tier, with the cell; a cell that ended
-            // inconsistent after such a test, or that the record cannot hold,
-            // goes to the FP64 twin instead
-            const uint32_t nt = active && !g.overflow ? g.S->ntent : 0u;
-            if (nt > 0u && g.status == kInconsistentBoundary) {
-                g.overflow = true, g.bail = 1u;
-            } else if (nt > 0u) {
-                // (the base comes from the group's lane 0 through a shuffle:
-                // a store and load of one LDS word by different lanes are not
-                // ordered for the compiler)
-                uint32_t base = 0u;
-                if (g.gl == 0) base = atomicAdd(&P.counters[7], nt);
-                base = (uint32_t)g.gbi((int)base, 0);
-                const bool fits = (uint64_t)base + nt <= (uint64_t)P.tent_cap;
-                if ((uint32_t)g.gl < nt && (uint64_t)base + g.gl < (uint64_t)P.tent_cap) {
-                    uint32_t *rec = P.tent + 5 * ((uint64_t)base + g.gl);
-                    const uint32_t t = g.S->tent[g.gl][0];
-                    rec[0] = fits ? cell : kNoCell;
-                    rec[1] = __float_as_uint(g.S->plx[tri_get<T::kB>(t, 0)].y);
-                    rec[2] = __float_as_uint(g.S->plx[tri_get<T::kB>(t, 1)].y);
-                    rec[3] = __float_as_uint(g.S->plx[tri_get<T::kB>(t, 2)].y);
-                    rec[4] = g.S->tent[g.gl][1];
-                }
-                if (!fits) g.overflow = true, g.bail = 1u;
-            }
-        }
+        if (active && g.gl == 0 && g.S->exact_events) log_exact(P, orig, g.S->exact_events);
         const bool emit = active && !g.overflow;
         const int F = emit ? g.stage_row(P) : 0;
         // the wave's four rows, back to back in the wave's current pool chunk
@@ -1734,86 +1596,50 @@ __device__ __forceinline__ void tier0_body(const CellParams &prm) {
             }
         }
         uint32_t slot = 0u;
-        if (!emit && active && g.gl == 0) {
-            if (!kExactTier && g.bail) {  // flag for the FP64-capable instance
-                if (g.bail < 3u) g.count(g.bail == 1u ? kCtrBailTest : kCtrBailVertex);
-                P.exact_list[c] = 1u;
-                atomicAdd(&P.counters[5], 1u);
-            } else {  // queue for the large-capacity tier
-                g.count(kStatPromoted);
-                slot = atomicAdd(&P.counters[1], 1u);
-                if (slot < P.queue_cap) P.mid_list[slot] = cell;
-                else truncate_cell(P, orig);
-            }
+        if (!emit && active && g.gl == 0) {  // queue for the large-capacity tier
+            g.count(kStatPromoted);
+            slot = atomicAdd(&P.counters[1], 1u);
+            if (slot < P.queue_cap) P.mid_list[slot] = cell;
+            else truncate_cell(P, orig);
         }
         // with the promotion, the owners of the planes held (the large tier
         // starts from them); the slot comes from the group's lane 0
-        if (active && !emit && (kExactTier || !g.bail)) {
+        if (active && !emit) {
             slot = (uint32_t)g.gbi((int)slot, 0);
             if (slot < P.promo_cap) g.store_owners(P.promo + (size_t)slot * kPromoPlanes);
         }
         if (active && P.cycles && g.gl == 0) P.cycles[orig] = (uint32_t)min(clock64() - t0, (uint64_t)0x7fffffff);
-        if (active && g.gl == 0 && !g.bail) cells++;
+        if (active && g.gl == 0) cells++;
     };
-    if constexpr (!kExactTier) {
-        if (prm.clouds == nullptr) {
-            while (true) {
-                uint32_t c0 = 0;
-                if (lane == 0) c0 = atomicAdd(&prm.counters[0], (uint32_t)kCellsPerWave);
-                c0 = uniform(c0);
-                if ((int64_t)c0 >= count) break;
-                round((int64_t)c0 + grp < count, (int64_t)c0 + grp);
-            }
-        } else {
-            // a batch: one quad (four consecutive cells of one cloud) per round,
-            // so the cells of a wave share their cloud's subtree
-            const int64_t nq = prm.quads[prm.n_clouds];
-            while (true) {
-                uint32_t q0 = 0;
-                if (lane == 0) q0 = atomicAdd(&prm.counters[0], 1u);
-                const int64_t q = (int64_t)uniform(q0);
-                if (q >= nq) break;
-                const int cl = uniform(batch_find(prm.quads, prm.n_clouds, q));
+    while (true) {
+        uint32_t w = 0;
+        if (lane == 0) w = atomicAdd(&prm.counters[6], 1u);
+        const int64_t base = (int64_t)uniform(w) * kWave;
+        if (base >= count) break;
+        uint64_t bits = __ballot(base + lane < count && prm.exact_list[base + lane] != 0u);
+        // in a batch the cells of a round must share a cloud
+        const int lc = (prm.clouds != nullptr && base + lane < count)
+                           ? batch_find(prm.cloud_cells, prm.n_clouds, prm.begin + base + lane) : 0;
+        while (bits) {
+            uint64_t take = bits;
+            if (prm.clouds != nullptr) {
+                const int cl = uniform(rl(lc, (int)__builtin_ctzll(bits)));
                 g.set_cloud(&prm.clouds[cl]);
-                const int64_t lo = max(prm.cloud_cells[cl], prm.begin), hi = min(prm.cloud_cells[cl + 1], prm.end);
-                const int64_t cell = lo + kCellsPerWave * (q - prm.quads[cl]) + grp;
-                round(cell < hi, cell - prm.begin);
+                take = bits & __ballot(lc == cl);
             }
-        }
-    } else {
-        while (true) {
-            uint32_t w = 0;
-            if (lane == 0) w = atomicAdd(&prm.counters[6], 1u);
-            const int64_t base = (int64_t)uniform(w) * kWave;
-            if (base >= count) break;
-            uint64_t bits = __ballot(base + lane < count && prm.exact_list[base + lane] != 0u);
-            // in a batch the cells of a round must share a cloud
-            const int lc = (prm.clouds != nullptr && base + lane < count)
-                               ? batch_find(prm.cloud_cells, prm.n_clouds, prm.begin + base + lane) : 0;
-            while (bits) {
-                uint64_t take = bits;
-                if (prm.clouds != nullptr) {
-                    const int cl = uniform(rl(lc, (int)__builtin_ctzll(bits)));
-                    g.set_cloud(&prm.clouds[cl]);
-                    take = bits & __ballot(lc == cl);
-                }
-                uint64_t b = take;  // the grp-th flagged cell of the round
-                for (int t = 0; t < grp; ++t) b &= b - 1ull;
-                uint64_t used = take;
-                for (int t = 0; t < kCellsPerWave; ++t) used &= used - 1ull;
-                bits &= ~(take & ~used);
-                round(b != 0ull, base + (b ? (int64_t)__builtin_ctzll(b) : 0));
-            }
+            uint64_t b = take;  // the grp-th flagged cell of the round
+            for (int t = 0; t < grp; ++t) b &= b - 1ull;
+            uint64_t used = take;
+            for (int t = 0; t < kCellsPerWave; ++t) used &= used - 1ull;
+            bits &= ~(take & ~used);
+            round(b != 0ull, base + (b ? (int64_t)__builtin_ctzll(b) : 0));
         }
     }
     g.flush(prm, cells);
 }
 
-__global__ void __launch_bounds__(kT0Threads) __attribute__((amdgpu_waves_per_eu(3, 3))) cell_group_kernel(const CellParams prm) {
-    tier0_body<Tier0, false>(prm);
-}
 __global__ void __launch_bounds__(kT0Threads) cell_group_exact_kernel(const CellParams prm) {
-    tier0_body<Tier0x, true>(prm);
+    tier0x_body<Tier0x>(prm);
 }
 // The same at 3 waves per SIMD, as tier 0, for batches of clouds, where many
 // cells come here (a fifth of a LiDAR batch): the third wave gains more than
@@ -1821,7 +1647,7 @@ __global__ void __launch_bounds__(kT0Threads) cell_group_exact_kernel(const Cell
 // every persistent wave writes its spills once, so it keeps the uncapped one.
 __global__ void __launch_bounds__(kT0Threads) __attribute__((amdgpu_waves_per_eu(3, 3)))
 cell_group_exact_batch_kernel(const CellParams prm) {
-    tier0_body<Tier0x, true>(prm);
+    tier0x_body<Tier0x>(prm);
 }
 
 // Decides in FP64 (where FP64 cannot, exactly) the removal tests tier 0 took

@@ -9,6 +9,7 @@
 // so no primitive-id indirection is needed.
 #include "pg_common.hpp"
 #include "pg_kernels.hpp"
+#include "pg_wide.hpp"
 
 #include <float.h>
 
@@ -390,6 +391,27 @@ __global__ void refit_top_kernel(const float4 *__restrict__ pts, int64_t n, cons
     }
 }
 
+// The 16-wide form (pg_wide.hpp), one thread per binary node; the few that
+// are maximal in their class fill a record.  In a batch (cloud_shift < 32:
+// the keys' leading bits name the cloud) each cloud has its own wide form.
+__global__ void wide_kernel(const Node *__restrict__ nodes, int64_t n, const uint32_t *__restrict__ parents,
+                            const uint2 *__restrict__ ranges, const uint32_t *__restrict__ keys, int cloud_shift,
+                            WideChild *__restrict__ wide) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n - 1) return;
+    const uint2 r = ranges[i];
+    const int k = wide_class(r.y - r.x + 1u);
+    if (k == 0) return;
+    auto crosses = [&](uint2 q) { return cloud_shift < 32 && ((keys[q.x] ^ keys[q.y]) >> cloud_shift) != 0u; };
+    const uint32_t p = parents[i];
+    if (p != 0xFFFFFFFFu) {
+        const uint2 q = ranges[p];
+        if (wide_class(q.y - q.x + 1u) == k && !crosses(q)) return;
+    }
+    if (crosses(r)) return;
+    wide_fill((uint32_t)i, k, (uint32_t)n, nodes, ranges, wide + 16ull * wide_slot((uint32_t)n, k, r.x));
+}
+
 // Points identical in position and weight have identical Morton keys, so
 // each duplicate group lies inside one run of equal keys: scan the run.
 // Groups of exact duplicates (equal position and weight) among the
@@ -555,9 +577,10 @@ hipError_t fill_u32(uint32_t *p, int64_t n, uint32_t v, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// Sort, hierarchy and refit over keys already written to the workspace.
-static hipError_t build_tail(int64_t n, const float *points, const float *weights, int leaf_size, char *base,
-                             const IndexLayout &L, hipStream_t stream) {
+// Sort, hierarchy, refit and wide form over keys already written to the
+// workspace (cloud_bits: the keys' leading bits that name the cloud).
+static hipError_t build_tail(int64_t n, const float *points, const float *weights, int leaf_size, int cloud_bits,
+                             char *base, const IndexLayout &L, hipStream_t stream) {
     IndexHeader *hdr = (IndexHeader *)(base + L.header);
     float4 *sorted = (float4 *)(base + L.points);
     uint32_t *perm = (uint32_t *)(base + L.perm);
@@ -613,6 +636,10 @@ static hipError_t build_tail(int64_t n, const float *points, const float *weight
         if (n > kRefitChunk)
             hipLaunchKernelGGL(refit_top_kernel, dim3(grid_for(n - 1, 256)), dim3(256), 0, stream, sorted, n, children,
                                parents, ranges, boxes, flags, nodes, leaf_size);
+        // the wide form takes the boxes' place
+        if (n > kWideLeaf)
+            hipLaunchKernelGGL(wide_kernel, dim3(grid_for(n - 1, 256)), dim3(256), 0, stream, nodes, n, parents, ranges,
+                               keys, 32 - cloud_bits, (WideChild *)boxes);
     }
     return hipGetLastError();
 }
@@ -641,7 +668,7 @@ hipError_t build_index(int64_t n, const float *points, const float *weights, int
                        weights ? 1 : 0, leaf_size);
     hipLaunchKernelGGL(morton_kernel, dim3(grid_for(n, 256)), dim3(256), 0, stream, points, n, hdr, keys);
 
-    return build_tail(n, points, weights, leaf_size, base, L, stream);
+    return build_tail(n, points, weights, leaf_size, 0, base, L, stream);
 }
 
 // ------------------------------------------------------------------ batches
@@ -772,7 +799,7 @@ hipError_t build_batch_index(int64_t n, int n_clouds, const float *points, const
                        n_clouds, weights ? 1 : 0, leaf_size, clouds, hdr, n);
     hipLaunchKernelGGL(batch_morton_kernel, dim3(grid_for(n, 256)), dim3(256), 0, stream, points, n, cloud_offsets,
                        n_clouds, clouds, batch_cloud_bits(n_clouds), batch_axis_bits(n_clouds), keys);
-    if (hipError_t e = build_tail(n, points, weights, leaf_size, base, L, stream)) return e;
+    if (hipError_t e = build_tail(n, points, weights, leaf_size, batch_cloud_bits(n_clouds), base, L, stream)) return e;
     hipLaunchKernelGGL(batch_roots_kernel, dim3(grid_for(n_clouds, 256)), dim3(256), 0, stream, n, cloud_offsets,
                        n_clouds, (const uint32_t *)(base + L.parents), (const uint2 *)(base + L.ranges), leaf_size, hdr,
                        clouds);
