@@ -1,8 +1,8 @@
 """The 16-wide form of the hierarchy against the CPU oracle, bit for bit, where
 it can go wrong: cloud sizes at the edges of its classes (32 * 8^k points), leaf
 sizes up to a whole class, a chain of clusters whose nodes have more than 16
-children (walked as binary nodes), and batches whose clouds lie in different
-classes.  Whole-number outputs: no tolerance."""
+children (walked as binary nodes), cells of many faces (built by the larger
+tiers, a wave per cell), and batches whose clouds lie in different classes.  Whole-number outputs: no tolerance."""
 import numpy as np
 import pytest
 
@@ -44,6 +44,19 @@ def test_more_than_16_children(gpu, per_cluster, rest):
     assert_matches_oracle(run(gpu, pts), pts)
     w = np.random.default_rng(5).uniform(0, 1e-7, pts.shape[0]).astype(np.float32)
     assert_matches_oracle(run(gpu, pts, w), pts, w)
+
+
+@pytest.mark.parametrize("faces", [40, 97, 98, 99, 130, 257, 258, 259, 500])
+def test_hub_cells(gpu, faces):
+    """A point amid ``faces`` points of a sphere: its cell has that many faces and
+    about twice the vertices, at the edges of the larger tiers' capacities."""
+    print(f"wide form: hub of {faces} faces", flush=True)
+    rng = np.random.default_rng(faces)
+    d = rng.standard_normal((faces, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    far = rng.random((1500, 3)) * 2.0 + 2.0
+    pts = np.concatenate([np.zeros((1, 3)), d, far]).astype(np.float32)
+    assert_matches_oracle(run(gpu, pts), pts)
 
 
 def test_batch_of_classes(gpu):
