@@ -85,6 +85,7 @@ struct CellParams {
     const int64_t *cloud_cells;   // [n_clouds + 1] sorted-cell range of each cloud
     const int64_t *quads;         // [n_clouds + 1] first work quad of each cloud within [begin, end)
     int n_clouds;
+    int cells_per_wave;           // of tier 0's small instance: groups of a wave that take a cell
     const float *init_h;          // optional [n] (original order): predicted half-width of each cell
     float *extent;                // optional [n] (original order): half-width of each built cell
 };
@@ -231,7 +232,15 @@ hipError_t launch_cells(const CellArgs &a, hipStream_t stream) {
     prm.promo_cap = (uint32_t)promo_slots(count);
     prm.tent = (uint32_t *)(sc + 256 + 16 * count + 4 * kPromoPlanes * promo_slots(count));
     prm.tent_cap = (uint32_t)tent_slots(count);
-    const int64_t cells_per_block = kT0Threads / kT0Lanes;
+    // A launch that cannot fill the chip (a.waves: 4 per SIMD, of which 3 are
+    // resident) lasts as long as its longest wave, and a wave as long as the
+    // longest of its cells: one cell per wave while that gives two waves per
+    // SIMD at most, two while all are resident at once.  Whole calls with four
+    // / two / one cells per wave: 1 k points 536 / 519 / 503 us, 2 k 607 / 596 /
+    // 595, 4 k 677 / 658 / 705, 6 k 759 / 720 / 773, 8 k 1023 / 1105 / 1153.
+    const bool small = prm.clouds == nullptr && count <= (int64_t)a.waves * 3 / 2;
+    prm.cells_per_wave = !small ? kWave / kT0Lanes : count <= a.waves / 2 ? 1 : 2;
+    const int64_t cells_per_block = prm.cells_per_wave * (kT0Threads / kWave);
     const int64_t blocks_needed = (count + cells_per_block - 1) / cells_per_block;
     const int64_t max_blocks = (int64_t)a.waves * kWave / kT0Threads;
     const int64_t blocks = max_blocks < blocks_needed ? max_blocks : blocks_needed;
@@ -246,7 +255,8 @@ hipError_t launch_cells(const CellArgs &a, hipStream_t stream) {
     }
     hipLaunchKernelGGL(cell_prep_kernel, dim3(1), dim3(64), 0, stream, prm.counters);
     if (hipError_t e = fill_u32(prm.exact_list, count, 0u, stream)) return e;
-    hipLaunchKernelGGL(cell_group_kernel, dim3((unsigned)(blocks > 0 ? blocks : 1)), dim3(kT0Threads), 0, stream, prm);
+    hipLaunchKernelGGL(small ? cell_group_small_kernel : cell_group_kernel, dim3((unsigned)(blocks > 0 ? blocks : 1)),
+                       dim3(kT0Threads), 0, stream, prm);
     {
         const uint64_t want = ((uint64_t)prm.tent_cap + 255) / 256;
         hipLaunchKernelGGL(cell_tentative_check_kernel, dim3((unsigned)(want < 2048 ? want : 2048)), dim3(256), 0,

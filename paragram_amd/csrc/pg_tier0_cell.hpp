@@ -856,8 +856,8 @@ struct Tier0 {
                     const float4 chi = make_float4(gbf(hi.x, c), gbf(hi.y, c), gbf(hi.z, c), 0.0f);
                     const bool pass = !balls_clear(clo, chi);
                     left = look ? left & ~(1u << c) : left;
-                    key = look & (gl == c) ? FLT_MAX : key;
-                    r = look & pass ? rc : r;
+                    key = (look & (gl == c)) ? FLT_MAX : key;
+                    r = (look & pass) ? rc : r;
                     visit |= look & pass;
                     look &= !pass & (left != 0u);
                 }
@@ -869,9 +869,9 @@ struct Tier0 {
                 uint32_t up_node, up_left;
                 pop(sz > 0 ? sz - 1 : 0, up_node, up_left);
                 push(keep, sz, node, left);
-                sz += keep ? 1 : (back & !end ? -1 : 0);
-                node = down ? r : (back & !end ? up_node : node);
-                left = down ? 0xFFFFu : (back & !end ? up_left : left);
+                sz += keep ? 1 : ((back & !end) ? -1 : 0);
+                node = down ? r : ((back & !end) ? up_node : node);
+                left = down ? 0xFFFFu : ((back & !end) ? up_left : left);
                 fresh = !(down | back);
                 base = leaf ? leaf_first(r) : base;
                 n = leaf ? (int)leaf_count(r) : n;
@@ -1098,9 +1098,11 @@ struct Tier0 {
 };
 
 // Tier 0's waves take Morton-consecutive quads of cells from a global
-// counter (a batch's quads each lie in one cloud).  A cell the tier gives up
+// counter (a batch's quads each lie in one cloud; kSmall: cells_per_wave cells
+// of one cloud, see launch_cells).  A cell the tier gives up
 // on (`bail`) is flagged for its FP64-capable twin; one that outgrows it is
 // queued for tier m.
+template <bool kSmall>
 __device__ __forceinline__ void tier0_body(const CellParams &prm) {
     constexpr int kCellsPerWave = kWave / kT0Lanes;
     __shared__ Tier0::LDS lds[kT0Threads / kT0Lanes];
@@ -1126,7 +1128,10 @@ __device__ __forceinline__ void tier0_body(const CellParams &prm) {
         if (lane == 0) k = atomicAdd(&prm.counters[0], 1u);
         const int64_t quad = (int64_t)uniform(k);
         int64_t c = kCellsPerWave * quad + grp, last = count;  // the group's cell, from prm.begin
-        if (prm.clouds == nullptr) {
+        if (kSmall) {
+            c = grp < prm.cells_per_wave ? prm.cells_per_wave * quad + grp : count;
+            if (prm.cells_per_wave * quad >= count) break;
+        } else if (prm.clouds == nullptr) {
             if (kCellsPerWave * quad >= count) break;
         } else {
             // a batch: the quad's cells share their cloud's subtree
@@ -1229,7 +1234,12 @@ __device__ __forceinline__ void tier0_body(const CellParams &prm) {
 }
 
 __global__ void __launch_bounds__(kT0Threads) __attribute__((amdgpu_waves_per_eu(3, 3))) cell_group_kernel(const CellParams prm) {
-    tier0_body(prm);
+    tier0_body<false>(prm);
+}
+// An instance of its own: the choice made in the kernel above costs it 0.7%.
+__global__ void __launch_bounds__(kT0Threads) __attribute__((amdgpu_waves_per_eu(3, 3)))
+cell_group_small_kernel(const CellParams prm) {
+    tier0_body<true>(prm);
 }
 
 }  // namespace pg

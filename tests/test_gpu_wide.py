@@ -37,6 +37,14 @@ def test_class_edges(gpu, n, leaf):
     assert_matches_oracle(run(gpu, pts, leaf_size=leaf), pts)
 
 
+@pytest.mark.parametrize("n", [3, 5, 4095, 4096, 4097, 6143, 6144, 6145])
+def test_cells_per_wave_edges(gpu, n):
+    """Sizes at which a wave takes one, two or four cells (2048 is among the above)."""
+    print(f"cells per wave: n={n}", flush=True)
+    pts = workloads.uniform(n, 300 + n)
+    assert_matches_oracle(run(gpu, pts), pts)
+
+
 @pytest.mark.parametrize("per_cluster,rest", [(20, 300), (1, 40), (70, 2100)])
 def test_more_than_16_children(gpu, per_cluster, rest):
     pts = chain(per_cluster, rest)
