@@ -391,25 +391,88 @@ __global__ void refit_top_kernel(const float4 *__restrict__ pts, int64_t n, cons
     }
 }
 
-// The 16-wide form (pg_wide.hpp), one thread per binary node; the few that
-// are maximal in their class fill a record.  In a batch (cloud_shift < 32:
-// the keys' leading bits name the cloud) each cloud has its own wide form.
-__global__ void wide_kernel(const Node *__restrict__ nodes, int64_t n, const uint32_t *__restrict__ parents,
-                            const uint2 *__restrict__ ranges, const uint32_t *__restrict__ keys, int cloud_shift,
-                            WideChild *__restrict__ wide) {
+// The 16-wide form (pg_wide.hpp).  One lane per binary node finds the few that
+// are maximal in their class; the 16 lanes of a group then fill the record of
+// one of them together, a child per lane, splitting every child that is too
+// large at once while lanes are left: 3 or 4 rounds of loads, where a thread
+// that split one child after the other took 14.  In a batch (cloud_shift < 32: the keys' leading bits name the
+// cloud) each cloud has its own wide form.
+__global__ void __launch_bounds__(256) wide_kernel(const Node *__restrict__ nodes, int64_t n,
+                                                   const uint32_t *__restrict__ parents,
+                                                   const uint2 *__restrict__ ranges, const uint32_t *__restrict__ keys,
+                                                   int cloud_shift, WideChild *__restrict__ wide) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n - 1) return;
-    const uint2 r = ranges[i];
-    const int k = wide_class(r.y - r.x + 1u);
-    if (k == 0) return;
+    const int lane = threadIdx.x & 63, gl = lane & 15, grp = lane >> 4;
     auto crosses = [&](uint2 q) { return cloud_shift < 32 && ((keys[q.x] ^ keys[q.y]) >> cloud_shift) != 0u; };
-    const uint32_t p = parents[i];
-    if (p != 0xFFFFFFFFu) {
-        const uint2 q = ranges[p];
-        if (wide_class(q.y - q.x + 1u) == k && !crosses(q)) return;
+    int k = 0;  // class of the lane's node if it gets a record
+    uint32_t first = 0u;
+    if (i < n - 1) {
+        const uint2 r = ranges[i];
+        k = wide_class(r.y - r.x + 1u);
+        first = r.x;
+        const uint32_t p = k != 0 ? parents[i] : 0xFFFFFFFFu;
+        if (p != 0xFFFFFFFFu) {
+            const uint2 q = ranges[p];
+            if (wide_class(q.y - q.x + 1u) == k && !crosses(q)) k = 0;
+        }
+        if (k != 0 && crosses(r)) k = 0;
     }
-    if (crosses(r)) return;
-    wide_fill((uint32_t)i, k, (uint32_t)n, nodes, ranges, wide + 16ull * wide_slot((uint32_t)n, k, r.x));
+    for (uint64_t todo = __ballot(k != 0); todo != 0ull;) {
+        // the group's node: the grp-th of those left
+        uint64_t m = todo;
+        for (int t = 0; t < 4; ++t) {
+            if (t < grp) m &= m - 1ull;
+            todo &= todo - 1ull;  // (0 stays 0)
+        }
+        const bool have = m != 0ull;
+        const int src = have ? (int)__builtin_ctzll(m) : 0;
+        const int kk = __shfl(k, src);
+        const uint32_t first_k = (uint32_t)__shfl((int)first, src);
+        const uint32_t top = (uint32_t)(i - lane + src);
+        const uint32_t limit = have ? wide_least(kk) - 1u : 0u;  // children have at most this many points
+        float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
+        uint32_t ref = kWideNone, at = 0u, size = 0u;  // child: binary reference, first point, points
+        auto take = [&](uint32_t parent, int side) {
+            const Node *nd = &nodes[parent];
+            lo = side ? nd->lo1 : nd->lo0;
+            hi = side ? nd->hi1 : nd->hi0;
+            ref = __float_as_uint(hi.w);
+            if (is_leaf(ref)) {
+                at = leaf_first(ref);
+                size = leaf_count(ref);
+            } else {
+                const uint2 r = ranges[ref];
+                at = r.x;
+                size = r.y - r.x + 1u;
+            }
+        };
+        if (have && gl < 2) take(top, gl);
+        int held = have ? 2 : 16;
+        while (true) {
+            // the first children over the limit for which a lane is left split
+            const uint32_t over = (uint32_t)(__ballot(size > limit) >> (16 * grp)) & 0xFFFFu;
+            const int rank = __popc(over & ((1u << gl) - 1u));
+            const bool split = size > limit && rank < 16 - held;
+            if (__ballot(split) == 0ull) break;
+            const int splits = min(__popc(over), 16 - held);
+            // lane held + t takes the second half of the t-th of them
+            uint32_t from = over;
+            for (int t = 0; t < gl - held; ++t) from &= from - 1u;
+            const bool fresh = gl >= held && gl < held + splits;
+            const uint32_t parent = (uint32_t)__shfl((int)ref, fresh ? (int)__builtin_ctz(from) : gl, 16);
+            if (split || fresh) take(parent, fresh ? 1 : 0);
+            held += splits;
+        }
+        if (have) {
+            if (gl >= held) ref = kWideNone;
+            else if (size <= limit) ref = wide_ref((uint32_t)n, at, size);
+            else ref |= kWideBinary;  // its own binary node
+            hi.w = __uint_as_float(ref);
+            WideChild *out = wide + 16ull * wide_slot((uint32_t)n, kk, first_k) + gl;
+            out->lo = lo;
+            out->hi = hi;
+        }
+    }
 }
 
 // Points identical in position and weight have identical Morton keys, so
