@@ -11,6 +11,7 @@ constexpr int kDppXor1 = 0xB1;   // quad_perm [1, 0, 3, 2]
 constexpr int kDppXor2 = 0x4E;   // quad_perm [2, 3, 0, 1]
 constexpr int kDppRor4 = 0x124;  // row_ror:4
 constexpr int kDppRor8 = 0x128;  // row_ror:8
+constexpr int kDppLast = 0x15F;  // row_newbcast:15
 constexpr int kDppShr1 = 0x111, kDppShr2 = 0x112, kDppShr4 = 0x114, kDppShr8 = 0x118;  // row_shr:n
 
 template <int C>

@@ -130,7 +130,7 @@ struct Tier0 {
     // exclusive prefix sum over the group; total in `tot`
     __device__ __forceinline__ int gexcl(int x, int &tot) const {
         const int incl = row_scan(x);
-        tot = row_sum(x);
+        tot = dpp<kDppLast>(incl);
         return incl - x;
     }
     // ---------------------------------------------------------- vertices
@@ -387,9 +387,12 @@ struct Tier0 {
         // sends the cell to the FP64-capable tiers if the sign was wrong.
         const float pa1 = fabsf(q.x) + fabsf(q.y) + fabsf(q.z);
         const float c2 = fmaf(kG32, plane_perm(q), kTiny32);
-        bool mine[kRows], open = false;
-#pragma unroll
-        for (int k = 0; k < kRows; ++k) mine[k] = false;
+        // the removed vertices: bit v of the pair (the group's four rows; a
+        // flag per row and lane instead is packed into bytes and unpacked:
+        // 1.4% of the kernel, with the edges' places below from three ballots)
+        uint32_t rem0 = 0u, rem1 = 0u;
+        auto mine = [&](int k) { return (((k < 2 ? rem0 : rem1) >> (gl + 16 * (k & 1))) & 1u) != 0u; };
+        bool open = false;
 #pragma unroll
         for (int k = 0; k < kRows; ++k) {
             if (__ballot(nv > G * k) == 0ull) break;
@@ -397,7 +400,9 @@ struct Tier0 {
             const float Pv = fmaf(q.x, p.x, fmaf(q.y, p.y, fmaf(q.z, p.z, -q.w)));
             const float err = fmaf(pa1, p.w, c2);
             const bool in = gl + G * k < nv;
-            mine[k] = in & (Pv > 0.0f);  // (of a decided test; of an open one its FP32 sign)
+            const uint32_t bits = gballot(in & (Pv > 0.0f));  // (of a decided test; of an open one its FP32 sign)
+            if (k < 2) rem0 |= bits << (16 * (k & 1));
+            else rem1 |= bits << (16 * (k & 1));
             open |= in & !(fabsf(Pv) > err);
         }
         if (gany(open)) {  // (rare)
@@ -420,25 +425,25 @@ struct Tier0 {
             for (int k = 0; k < kRows; ++k) {
                 if ((unsure >> k) & 1u) {
                     S->tent[r][0] = S->vtri[gl + G * k];
-                    S->tent[r][1] = (uint32_t)owner | (mine[k] ? 0x80000000u : 0u);
+                    S->tent[r][1] = (uint32_t)owner | (mine(k) ? 0x80000000u : 0u);
                     ++r;
                 }
             }
             S->ntent = n0 + (uint32_t)tot;
         }
-        // the removed vertices, listed in tmp[0, R) in slot order
-        int R = 0;
+        const int R = __popc(rem0) + __popc(rem1);
+        if (R == 0) return false;  // the plane does not cut
+        // listed in tmp[0, R) in slot order
 #pragma unroll
         for (int k = 0; k < kRows; ++k) {
             if (__ballot(nv > G * k) == 0ull) break;
-            const uint32_t bits = gballot(mine[k]);
-            if (mine[k]) {
+            if (mine(k)) {
                 const int v = gl + G * k;
-                S->tmp[R + grank(bits)] = S->vtri[v] | ((uint32_t)v << kSlotShift);
+                const uint32_t lower = k & 1 ? ~(0xFFFF0000u << gl) : (1u << gl) - 1u;
+                const int at = k < 2 ? __popc(rem0 & lower) : __popc(rem0) + __popc(rem1 & lower);
+                S->tmp[at] = S->vtri[v] | ((uint32_t)v << kSlotShift);
             }
-            R += __popc(bits);
         }
-        if (R == 0) return false;  // the plane does not cut
         if (R == nv) {  // voronoi_convex_cell.cuh:430-435
             empty_cell();
             return true;
@@ -506,21 +511,21 @@ struct Tier0 {
                 }
             }
             const bool e0 = has_tri & !tw0, e1 = has_tri & !tw1, e2 = has_tri & !tw2;
-            const uint32_t b0 = gballot(e0), b1 = gballot(e1), b2 = gballot(e2);
-            const int n0 = __popc(b0), n1 = n0 + __popc(b1);
-            nb = n1 + __popc(b2);
+            int j = gexcl((int)e0 + (int)e1 + (int)e2, nb);
             const int x0 = (int)(t0 * t0), x1 = (int)(t1 * t1), x2 = (int)(t2 * t2);
             cycle = (e0 ? x0 - x1 : 0) + (e1 ? x1 - x2 : 0) + (e2 ? x2 - x0 : 0);
             // (every lane has read its triangle above)
-            if (e0) S->tmp[grank(b0)] = t0 | (t1 << kB);
-            if (e1) S->tmp[n0 + grank(b1)] = t1 | (t2 << kB);
-            if (e2) S->tmp[n1 + grank(b2)] = t2 | (t0 << kB);
+            if (e0) S->tmp[j] = t0 | (t1 << kB);
+            j += (int)e0;
+            if (e1) S->tmp[j] = t1 | (t2 << kB);
+            j += (int)e1;
+            if (e2) S->tmp[j] = t2 | (t0 << kB);
         } else {
             // clips that remove more triangles than the group has lanes: each
             // lane walks its own removed rows; an edge keeps the slot listed
             // in its word
             uint32_t emask = 0;
-            boundary_rows(mine, R, emask, cycle);
+            boundary_rows(rem0, rem1, R, emask, cycle);
             int j = gexcl(__popc(emask), nb);
             // (a removed set of R triangles without gaps has at most R + 2
             // boundary edges; more than tmp holds are never written)
@@ -560,7 +565,7 @@ struct Tier0 {
 #pragma unroll
             for (int k = 0; k < kRows; ++k) {
                 const int v = gl + G * k;
-                const bool mv = nb < R && v >= kept + nb && v < nv && !mine[k];
+                const bool mv = nb < R && v >= kept + nb && v < nv && !mine(k);
                 const uint32_t bits = gballot(mv);
                 if (mv) {
                     const uint32_t w = S->tmp[m + grank(bits)];
@@ -584,10 +589,11 @@ struct Tier0 {
 
     // Boundary edges of the lane's own removed rows: bit 3k + e of emask marks
     // edge e of row k.
-    __device__ __forceinline__ void boundary_rows(const bool (&mine)[kRows], int R, uint32_t &emask, int &cycle) const {
+    __device__ __forceinline__ void boundary_rows(uint32_t rem0, uint32_t rem1, int R, uint32_t &emask,
+                                                  int &cycle) const {
 #pragma unroll
         for (int k = 0; k < kRows; ++k) {
-            if (!mine[k]) continue;
+            if ((((k < 2 ? rem0 : rem1) >> (gl + 16 * (k & 1))) & 1u) == 0u) continue;
             const uint32_t t = S->vtri[gl + G * k];
             const uint32_t t0 = tri_get<kB>(t, 0), t1 = tri_get<kB>(t, 1), t2 = tri_get<kB>(t, 2);
             bool tw0 = false, tw1 = false, tw2 = false;
