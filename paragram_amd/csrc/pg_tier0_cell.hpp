@@ -33,7 +33,7 @@
 // mask, both children of a node tested by every lane), one group walking the
 // 16-wide form for itself visits a tenth of the nodes, and its lanes test
 // different boxes: 8.1e9 instructions in place of 10.2e9 on 1 M uniform
-// points, and the tier takes 15.7 ms in place of 20.2.  The exact ball test
+// points, and the tier took 15.7 ms in place of 20.2 (14.6 with the later steps).  The exact ball test
 // of a child is put off until the walk comes to it, and is done by the whole
 // group, a vertex per lane: testing it for each child by that child's lane
 // took 23.7 ms.  The walk itself is written as selects in one loop that the
