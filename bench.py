@@ -51,9 +51,8 @@ WORKLOADS = {
            "{total:,} points in all), seed {seed}, one launch"),
 }
 TRAFFIC_PATH = os.path.join(ROOT, "profiles", "cell_kernel_traffic.json")
-CELL_KERNELS = ("cell_group_kernel", "cell_tentative_check_kernel", "cell_group_exact_kernel",
-                "cell_group_exact_batch_kernel", "cell_group_mid_kernel", "cell_group_big_kernel",
-                "cell_group_huge_kernel")  # (the FP64 twin's batch form launches for batches)
+CELL_KERNELS = ("cell_group_kernel", "cell_tentative_check_kernel", "cell_flagged_kernel",
+                "cell_group_mid_kernel", "cell_group_big_kernel", "cell_group_huge_kernel")
 COPY_KERNEL = "__amd_rocclr_copyBuffer"
 
 
@@ -468,9 +467,7 @@ def main() -> int:
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 5),
                      "traffic": traffic,
-                     "kernel": "cell construction: pg::" + " + pg::".join(
-                         k for k in CELL_KERNELS if k != ("cell_group_exact_kernel" if clouds is not None
-                                                          else "cell_group_exact_batch_kernel")),
+                     "kernel": "cell construction: pg::" + " + pg::".join(CELL_KERNELS),
                      "kernel_ms": round(kern_s * 1e3, 4),
                      "bytes_per_cell": round(b_cell, 2)},
         "cpu_baseline": cpu,

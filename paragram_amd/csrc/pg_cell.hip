@@ -175,7 +175,7 @@ __global__ void cell_prep_kernel(uint32_t *counters) {
 // queue can fill), the plane owners of the first cells queued for tier m
 // (room for one cell in 32, and 64 more; a cell past them starts without) and
 // the removal tests tier 0 took by their FP32 sign (room for one test per two
-// cells, and 1024 more; a cell past them goes to the FP64 twin).
+// cells, and 1024 more; a cell past them goes to tier m).
 uint64_t promo_slots(int64_t cells) { return (uint64_t)cells / 32 + 64; }
 uint64_t tent_slots(int64_t cells) { return (uint64_t)cells / 2 + 1024; }
 uint64_t cell_scratch_bytes(int64_t cells) {
@@ -246,8 +246,7 @@ hipError_t launch_cells(const CellArgs &a, hipStream_t stream) {
     const int64_t blocks = max_blocks < blocks_needed ? max_blocks : blocks_needed;
     // A tier-0 wave takes the pool in chunks, one device-wide atomic per
     // several rounds; what the waves of tier 0 leave unused is at most 1/16
-    // of the pool, and as much again for its FP64 twin (same grid, same
-    // chunks).  A pool that runs short is reported and grown, never silent.
+    // of the pool.  A pool that runs short is reported and grown, never silent.
     {
         const uint64_t waves0 = (uint64_t)(blocks > 0 ? blocks : 1) * (kT0Threads / kWave);
         const uint64_t per_wave = prm.rows_elems / (16 * waves0);
@@ -262,12 +261,10 @@ hipError_t launch_cells(const CellArgs &a, hipStream_t stream) {
         hipLaunchKernelGGL(cell_tentative_check_kernel, dim3((unsigned)(want < 2048 ? want : 2048)), dim3(256), 0,
                            stream, prm);
     }
-    if (prm.clouds != nullptr)
-        hipLaunchKernelGGL(cell_group_exact_batch_kernel, dim3((unsigned)(blocks > 0 ? blocks : 1)), dim3(kT0Threads),
-                           0, stream, prm);
-    else
-        hipLaunchKernelGGL(cell_group_exact_kernel, dim3((unsigned)(blocks > 0 ? blocks : 1)), dim3(kT0Threads), 0,
-                           stream, prm);
+    {
+        const int64_t want = (count + 255) / 256;
+        hipLaunchKernelGGL(cell_flagged_kernel, dim3((unsigned)(want < 2048 ? want : 2048)), dim3(256), 0, stream, prm);
+    }
     // tier m keeps 12 waves per CU resident where tier 1 keeps 8
     hipLaunchKernelGGL(cell_group_mid_kernel, dim3((unsigned)(a.waves1 * 3 / 2 * kWave / kTmThreads)),
                        dim3(kTmThreads), 0, stream, prm);

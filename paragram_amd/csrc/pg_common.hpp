@@ -59,19 +59,15 @@ enum StatSlot : int {
     kStatBailVertex = 25,    // ... a new vertex whose FP32 orientation was not safely positive
     kStatTentative = 26,     // removal tests tier 0 took by their FP32 sign (decided in FP64 after it)
     kStatTentativeWrong = 27,  // ... whose FP64 decision differed (or whose vertex lay on a predicted
-                               // cube's plane): the cell was rebuilt by the FP64 twin
+                               // cube's plane): the cell was rebuilt by tier m
     kStatTentativeLog = 28,  // 28..31: original ids of the first such cells, plus 1
     kNumStats = 32,
 };
 constexpr int kTentativeLogSlots = 4;
 // Removal tests one tier-0 cell may take by their FP32 sign (kept in LDS
-// until the cell is written out); a cell with more goes to the FP64 twin.
+// until the cell is written out); a cell with more goes to tier m.
 constexpr int kTentMax = 8;
 constexpr uint32_t kNoCell = 0xFFFFFFFFu;  // a record slot that holds no test
-// Up to this many cells flagged for the FP64-capable tier 0 go to tier m's
-// queue instead (tier m builds them beside its own; the twin's launch would
-// last as long as its slowest cell for a handful of cells).
-constexpr uint32_t kFewFlagged = 2048;
 constexpr int kExactLogSlots = 7;
 constexpr int kPromoPlanes = 48;  // plane owners kept for a cell promoted to tier m (tier 0's plane capacity)
 // Statistics first summed per group in LDS: slots 0..11, then the two bail

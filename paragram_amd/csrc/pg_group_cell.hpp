@@ -1140,125 +1140,14 @@ struct Group {
         }
     }
 
-    // ---------------------------------------------------------- wait list
-    // Depth-first wait list (a stack) shared by the cells of one wave, in
-    // registers: entry t sits in slot t / 64 of lane t % 64.  Entries are
-    // parent << 1 | child.
-    __device__ __forceinline__ void list_push(int t, uint32_t e) {
-        const bool me = lane64 == (t & (kWave - 1));
-        const int sl = t / kWave;
-#pragma unroll
-        for (int j = 0; j < kLS; ++j) lr[j] = (me && j == sl) ? e : lr[j];
-    }
-    __device__ __forceinline__ uint32_t list_pop(int &sz) {
-        const int t = --sz;
-        uint32_t r = 0u;
-#pragma unroll
-        for (int j = 0; j < kLS; ++j) r = j == t / kWave ? lr[j] : r;
-        return rl(r, t & (kWave - 1));
-    }
-
-    // Wave-wide: does any cell of the wave still need this box?  key: the
-    // smallest bound over the cells that need it; mine: this cell needs it.
-    __device__ __forceinline__ bool packet_needs(float4 lo, float4 hi, float &key, bool &mine) const {
-        float k = FLT_MAX;
-        const bool need = live() && !node_prunable<false>(lo, hi, k);
-        mine = need;
-        const bool any = __ballot(gl == 0 && need) != 0ull;
-        float kk = need ? k : FLT_MAX;
-        if constexpr (G == 16) kk = fminf(fminf(rl(kk, 0), rl(kk, 16)), fminf(rl(kk, 32), rl(kk, 48)));
-        key = uniform(kk);
-        return any;
-    }
-
-    // Both children of a node at once: the low half of each group tests
-    // child 0, the high half child 1.
-    __device__ __forceinline__ void packet_needs2(const Node &nd, bool &n0, bool &n1, float &k0, float &k1, bool &m0,
-                                                  bool &m1) const {
-        constexpr int H = G / 2;
-        const bool second = gl >= H;
-        const float4 lo = second ? nd.lo1 : nd.lo0, hi = second ? nd.hi1 : nd.hi0;
-        float k = FLT_MAX;
-        const bool need = live() && !node_prunable<true>(lo, hi, k);
-        const uint64_t b = __ballot(need);
-        m0 = ((b >> gshift) & 1ull) != 0ull;
-        m1 = ((b >> (gshift + H)) & 1ull) != 0ull;
-        constexpr uint64_t kLead = G == 16 ? 0x0001000100010001ull : 1ull;  // lane 0 of each group
-        n0 = (b & kLead) != 0ull;
-        n1 = (b & (kLead << H)) != 0ull;
-        const float kk = need ? k : FLT_MAX;
-        if constexpr (G == 16) {
-            k0 = uniform(fminf(fminf(rl(kk, 0), rl(kk, 16)), fminf(rl(kk, 32), rl(kk, 48))));
-            k1 = uniform(fminf(fminf(rl(kk, H), rl(kk, 16 + H)), fminf(rl(kk, 32 + H), rl(kk, 48 + H))));
-        } else {
-            k0 = uniform(rl(kk, 0));
-            k1 = uniform(rl(kk, H));
-        }
-    }
-
-    // Depth-first packet traversal: the cells of a wave (Morton neighbours)
-    // walk the hierarchy together.  A box is expanded while any of them may
-    // still be cut by a point in it; of two needed children the one with the
-    // smaller key (the smallest lower bound of H over the cells that need
-    // it) comes first and the other waits on a wave-wide stack, re-tested
-    // when it comes out.  A leaf goes only to the cells whose own test kept
-    // its box (the others could not be cut by its points).  The reference
-    // pops the smallest key instead (voronoi_bvh.cuh:246-283); after the kNN
-    // pre-clip the order changes little of the work and the stack needs no
-    // arg-min, and the diagram does not depend on it.  A full stack sends the
-    // wave's cells to the next tier instead of dropping entries.
-    __device__ __forceinline__ void traverse() {
-        uint32_t ref = uniform(root_ref);
-        int sz = 0;
-        bool mine = true;  // this cell needs box ref
-        while (true) {
-            bool have = false;
-            if (is_leaf(ref)) {
-                if (live() && mine) offer_leaf(ref);
-            } else {
-                if (lane64 == 0) count(kStatNodes);
-                const Node nd = nodes[ref];
-                float k0, k1;
-                bool m0, m1, n0, n1;
-                packet_needs2(nd, n0, n1, k0, k1, m0, m1);
-                const uint32_t r0 = uniform(__float_as_uint(nd.hi0.w)), r1 = uniform(__float_as_uint(nd.hi1.w));
-                if (n0 || n1) {
-                    const bool near0 = !n1 || (n0 && k0 <= k1);
-                    if (n0 && n1) {  // the farther child waits
-                        if (sz >= L) {
-                            overflow = true;
-                            return;
-                        }
-                        list_push(sz++, (ref << 1) | (near0 ? 1u : 0u));
-                    }
-                    ref = near0 ? r0 : r1;
-                    mine = near0 ? m0 : m1;
-                    have = true;
-                }
-            }
-            while (!have) {
-                if (sz == 0) return;
-                const uint32_t e = list_pop(sz);
-                const uint32_t parent = e >> 1, c = e & 1u;
-                const Node nd = nodes[parent];
-                float k;
-                const float4 lo = c ? nd.lo1 : nd.lo0;
-                const float4 hi = c ? nd.hi1 : nd.hi0;
-                if (packet_needs(lo, hi, k, mine)) {
-                    ref = uniform(__float_as_uint(hi.w));
-                    have = true;
-                }
-            }
-        }
-    }
-
+    // ---------------------------------------------------------- traversal
     // Depth-first walk of the wide form by a wave that builds one cell: lane
     // c < 16 holds child c of the node.  The children are tested against the
     // cell's octants by their lanes when the node is entered (and again when
     // the walk returns to it), and against the vertices by the whole wave one
     // at a time, nearest first, when the walk comes to them.  Every value that
     // steers it is uniform, and each step takes a child off a node's list.
-    __device__ __forceinline__ void traverse_wide() {
+    __device__ __forceinline__ void traverse() {
         uint32_t r = uniform(root_ref), node = 0u, left = 0u;
         int sz = 0;
         float4 lo, hi;
@@ -1555,7 +1444,6 @@ constexpr int kT0Lanes = 16, kT0Verts = 64, kT0Planes = 48, kT0List = 128, kT0Th
 constexpr int kTmLanes = 64, kTmVerts = 192, kTmPlanes = 128, kTmList = 128, kTmThreads = 128;
 constexpr int kT1Lanes = 64, kT1Verts = 512, kT1Planes = 255, kT1List = 128, kT1Threads = 128;
 constexpr int kT2Lanes = 64, kT2Verts = 1024, kT2Planes = 1023, kT2List = 128, kT2Threads = 64;
-using Tier0x = Group<kT0Lanes, kT0Verts, kT0Planes, kT0List>;
 using TierM = Group<kTmLanes, kTmVerts, kTmPlanes, kTmList>;
 using Tier1 = Group<kT1Lanes, kT1Verts, kT1Planes, kT1List>;
 using Tier2 = Group<kT2Lanes, kT2Verts, kT2Planes, kT2List>;
@@ -1600,144 +1488,26 @@ __device__ __forceinline__ uint64_t pool_take(const CellParams &P, uint32_t n) {
     return ((uint64_t)rl((uint32_t)(b >> 32), 0) << 32) | (uint64_t)rl((uint32_t)b, 0);
 }
 
-// Tier 0's twin: the waves scan the flags of the range in windows of 64
-// Morton-consecutive cells and take the flagged cells four at a time
-// (neighbours, so the shared traversal stays coherent).  A cell that outgrows
-// it is queued for tier m.
-template <typename T>
-__device__ __forceinline__ void tier0x_body(const CellParams &prm) {
-    constexpr int kCellsPerWave = kWave / kT0Lanes;
-    __shared__ GroupLDS<kT0Verts, kT0Planes> lds[kT0Threads / kT0Lanes];
-    __shared__ CandLDS<kT0Lanes> cands[kT0Threads / kT0Lanes];
-    __shared__ CellParams sprm;
-    // each wave's unused part of the row pool: next entry and entries left
-    __shared__ unsigned long long chunk_at[kT0Threads / kWave];
-    __shared__ uint32_t chunk_left[kT0Threads / kWave];
-    if (threadIdx.x == 0) sprm = prm;
-    if (threadIdx.x < kT0Threads / kWave) {
-        chunk_at[threadIdx.x] = 0ull;
-        chunk_left[threadIdx.x] = 0u;
-    }
-    __syncthreads();
-    const int lane = threadIdx.x & (kWave - 1);
-    const int grp = lane / kT0Lanes;
+// Queues the cells flagged by tier 0 and by the check of its recorded tests
+// for tier m, with no plane owners.  (An FP64 twin of tier 0, 16 lanes per
+// cell, rebuilt them before when more than 2048 were flagged; a wave per cell
+// is the faster of the two at every count: 500 k points with a predicted cube
+// 13.3 -> 12.1 ms, 100 k 5.3 -> 3.5, 2 M 50.7 -> 48.4, 640 k flagged cells of 256
+// LiDAR clouds 587 -> 571.)
+__global__ void __launch_bounds__(256) cell_flagged_kernel(const CellParams prm) {
     if (prm.counters[5] == 0u) return;  // no cell was flagged
-    if (prm.counters[5] <= kFewFlagged) {
-        // a few flagged cells: queued for tier m, with no plane owners (the
-        // flags read in a grid-stride loop: no work counter to contend for)
-        const int64_t count = prm.end - prm.begin;
-        const int64_t step = (int64_t)gridDim.x * kT0Threads;
-        for (int64_t c = (int64_t)blockIdx.x * kT0Threads + threadIdx.x; c < count; c += step) {
-            if (prm.exact_list[c] != 0u) {
-                const uint32_t slot = atomicAdd(&prm.counters[1], 1u);
-                const uint32_t cell = (uint32_t)(prm.begin + c);
-                if (slot < prm.queue_cap) prm.mid_list[slot] = cell;
-                else truncate_cell(prm, prm.perm[cell]);
-                if (slot < prm.promo_cap)
-                    for (int p = 0; p < kPromoPlanes; ++p) prm.promo[(size_t)slot * kPromoPlanes + p] = -1;
-            }
-        }
-        return;
-    }
-    T g;
-    g.setup(prm, &lds[(threadIdx.x / kWave) * kCellsPerWave + grp], &cands[(threadIdx.x / kWave) * kCellsPerWave + grp]);
-    uint32_t cells = 0;
     const int64_t count = prm.end - prm.begin;
-    // one round: cell begin + c for an active group
-    auto round = [&](bool active, int64_t c) {
-        const uint64_t t0 = clock64();
-        g.active = active;
-        const uint32_t cell = (uint32_t)(prm.begin + (active ? c : 0));
-        if (active) g.start(cell, *reread(&sprm));
-        g.traverse();
-        // the launch's fields again from the argument segment (scalar loads)
-        // rather than kept in registers across the traversal
-        const CellParams &P = *reread(&sprm);
-        const uint32_t orig = P.perm[cell];
-        if (active && g.gl == 0 && g.S->exact_events) log_exact(P, orig, g.S->exact_events);
-        const bool emit = active && !g.overflow;
-        const int F = emit ? g.stage_row(P) : 0;
-        // the wave's four rows, back to back in the wave's current pool chunk
-        const int f0 = rl(F, 0), f1 = rl(F, 16), f2 = rl(F, 32), f3 = rl(F, 48);
-        // (the chunk's position lives in LDS, not in registers across the traversal)
-        const uint32_t need = (uint32_t)(f0 + f1 + f2 + f3);
-        const int wv = threadIdx.x / kWave;
-        uint32_t left = uniform(chunk_left[wv]);
-        uint64_t at;
-        if (need > left) {
-            left = need > P.pool_chunk ? need : P.pool_chunk;
-            at = pool_take(P, left);
-        } else {
-            const unsigned long long a = chunk_at[wv];
-            at = ((uint64_t)uniform((uint32_t)(a >> 32)) << 32) | (uint64_t)uniform((uint32_t)a);
-        }
-        const uint64_t base = at + (uint64_t)(grp > 0 ? f0 : 0) + (uint64_t)(grp > 1 ? f1 : 0) +
-                              (uint64_t)(grp > 2 ? f2 : 0);
-        if (lane == 0) {
-            chunk_at[wv] = at + need;
-            chunk_left[wv] = left - need;
-        }
-        if (emit) {
-            if (base + (uint64_t)F <= P.rows_elems) {
-                if (g.gl == 0) P.row_offsets[cell] = (int64_t)base;
-                g.write_row(P, orig, P.rows + base, F);
-            } else if (g.gl == 0) {
-                pool_short(P, cell, orig, base + (uint64_t)F);
-            }
-        }
-        uint32_t slot = 0u;
-        if (!emit && active && g.gl == 0) {  // queue for the large-capacity tier
-            g.count(kStatPromoted);
-            slot = atomicAdd(&P.counters[1], 1u);
-            if (slot < P.queue_cap) P.mid_list[slot] = cell;
-            else truncate_cell(P, orig);
-        }
-        // with the promotion, the owners of the planes held (the large tier
-        // starts from them); the slot comes from the group's lane 0
-        if (active && !emit) {
-            slot = (uint32_t)g.gbi((int)slot, 0);
-            if (slot < P.promo_cap) g.store_owners(P.promo + (size_t)slot * kPromoPlanes);
-        }
-        if (active && P.cycles && g.gl == 0) P.cycles[orig] = (uint32_t)min(clock64() - t0, (uint64_t)0x7fffffff);
-        if (active && g.gl == 0) cells++;
-    };
-    while (true) {
-        uint32_t w = 0;
-        if (lane == 0) w = atomicAdd(&prm.counters[6], 1u);
-        const int64_t base = (int64_t)uniform(w) * kWave;
-        if (base >= count) break;
-        uint64_t bits = __ballot(base + lane < count && prm.exact_list[base + lane] != 0u);
-        // in a batch the cells of a round must share a cloud
-        const int lc = (prm.clouds != nullptr && base + lane < count)
-                           ? batch_find(prm.cloud_cells, prm.n_clouds, prm.begin + base + lane) : 0;
-        while (bits) {
-            uint64_t take = bits;
-            if (prm.clouds != nullptr) {
-                const int cl = uniform(rl(lc, (int)__builtin_ctzll(bits)));
-                g.set_cloud(prm, cl);
-                take = bits & __ballot(lc == cl);
-            }
-            uint64_t b = take;  // the grp-th flagged cell of the round
-            for (int t = 0; t < grp; ++t) b &= b - 1ull;
-            uint64_t used = take;
-            for (int t = 0; t < kCellsPerWave; ++t) used &= used - 1ull;
-            bits &= ~(take & ~used);
-            round(b != 0ull, base + (b ? (int64_t)__builtin_ctzll(b) : 0));
+    const int64_t step = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < count; c += step) {
+        if (prm.exact_list[c] != 0u) {
+            const uint32_t slot = atomicAdd(&prm.counters[1], 1u);
+            const uint32_t cell = (uint32_t)(prm.begin + c);
+            if (slot < prm.queue_cap) prm.mid_list[slot] = cell;
+            else truncate_cell(prm, prm.perm[cell]);
+            if (slot < prm.promo_cap)
+                for (int p = 0; p < kPromoPlanes; ++p) prm.promo[(size_t)slot * kPromoPlanes + p] = -1;
         }
     }
-    g.flush(prm, cells);
-}
-
-__global__ void __launch_bounds__(kT0Threads) cell_group_exact_kernel(const CellParams prm) {
-    tier0x_body<Tier0x>(prm);
-}
-// The same at 3 waves per SIMD, as tier 0, for batches of clouds, where many
-// cells come here (a fifth of a LiDAR batch): the third wave gains more than
-// the 76 registers it spills cost.  A single cloud sends few cells here, and
-// every persistent wave writes its spills once, so it keeps the uncapped one.
-__global__ void __launch_bounds__(kT0Threads) __attribute__((amdgpu_waves_per_eu(3, 3)))
-cell_group_exact_batch_kernel(const CellParams prm) {
-    tier0x_body<Tier0x>(prm);
 }
 
 // Decides in FP64 (where FP64 cannot, exactly) the removal tests tier 0 took
@@ -1820,7 +1590,7 @@ __device__ __forceinline__ void queued_tier_body(const CellParams &prm, const ui
         if constexpr (kOwners) {
             if (k < prm.promo_cap) g.offer_owners(prm.promo + (size_t)k * kPromoPlanes, kPromoPlanes);
         }
-        g.traverse_wide();
+        g.traverse();
         const CellParams &Q = *reread(&sprm);
         const uint32_t orig = Q.perm[cell];
         if (lane == 0 && g.S->exact_events) log_exact(Q, orig, g.S->exact_events);
@@ -1883,7 +1653,7 @@ __global__ void __launch_bounds__(kT2Threads) cell_group_huge_kernel(const CellP
         if (prm.clouds != nullptr) g.set_cloud(prm, uniform(batch_find(prm.cloud_cells, prm.n_clouds, cell)));
         g.active = true;
         g.start(cell, *reread(&sprm));
-        g.traverse_wide();
+        g.traverse();
         const CellParams &P = *reread(&sprm);
         const uint32_t orig = P.perm[cell];
         if (lane == 0 && g.S->exact_events) log_exact(P, orig, g.S->exact_events);

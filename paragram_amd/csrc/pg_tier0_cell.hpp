@@ -1106,8 +1106,7 @@ struct Tier0 {
 // Tier 0's waves take Morton-consecutive quads of cells from a global
 // counter (a batch's quads each lie in one cloud; kSmall: cells_per_wave cells
 // of one cloud, see launch_cells).  A cell the tier gives up
-// on (`bail`) is flagged for its FP64-capable twin; one that outgrows it is
-// queued for tier m.
+// on (`bail`) is flagged, one that outgrows it queued, for tier m.
 template <bool kSmall>
 __device__ __forceinline__ void tier0_body(const CellParams &prm) {
     constexpr int kCellsPerWave = kWave / kT0Lanes;
@@ -1162,7 +1161,7 @@ __device__ __forceinline__ void tier0_body(const CellParams &prm) {
         // the removal tests taken by their FP32 sign go to the record for the
         // FP64 check after this tier, with the cell; a cell that ended
         // inconsistent after such a test, or that the record cannot hold, goes
-        // to the FP64 twin instead
+        // to tier m instead
         const uint32_t nt = active && !g.overflow ? g.S->ntent : 0u;
         if (nt > 0u && g.status == kInconsistentBoundary) {
             g.overflow = true, g.bail = 1u;
@@ -1216,7 +1215,7 @@ __device__ __forceinline__ void tier0_body(const CellParams &prm) {
                 pool_short(P, cell, orig, base + (uint64_t)F);
             }
         } else if (active && g.gl == 0) {
-            if (g.bail) {  // flag for the FP64-capable twin
+            if (g.bail) {  // flag for tier m
                 if (g.bail < 3u) g.count(g.bail == 1u ? kCtrBailTest : kCtrBailVertex);
                 P.exact_list[c] = 1u;
                 atomicAdd(&P.counters[5], 1u);
