@@ -3,10 +3,7 @@
 // constants and the plane-triple helpers defined there), before
 // pg_tier0_cell.hpp, the FP32-only tier that every cell starts in.
 //
-// Four instances:
-//   tier 0's twin: G = 16 lanes, 64 vertex slots, 48 plane slots (about
-//           3.3 KB of LDS per cell, 4 cells per wave) -- the cells tier 0
-//           gave up on for their precision;
+// Three instances:
 //   tier m: G = 64 lanes, 192 vertex slots, 128 plane slots (one cell per
 //           wave, 12 waves per CU) -- the few cells that outgrow tier 0
 //           (cells with more than about 34 faces);
@@ -25,8 +22,6 @@
 //   plx[P]   float2  permanent of H and the owner (sorted point id, or a
 //                    negative box-plane code)
 //   tmp[V]   uint32  clip and emission scratch
-//   pm[P/2]  uint32  (16 lanes) per plane, a 16-bit mask of the lanes whose
-//                    removed triangle holds the plane; zero between clips
 // Vertices live in a pool of V slots with a group-uniform valid mask (slot
 // v = lane + G k belongs to lane v mod G), so a clip frees and refills slots
 // without moving data.
@@ -35,11 +30,9 @@
 // (one per lane, then offered in order), the boundary edges of a clip and
 // the new vertices they make, bounds reductions and the row sort.  All
 // control decisions are group-uniform (ballots restricted to the group).
-// The four cells of the twin's wave (Morton neighbours) share one depth-first
-// traversal of the binary hierarchy; the one cell of a larger tier's wave
-// walks the 16-wide form.
+// A wave walks the 16-wide form of the hierarchy for its one cell.
 //
-// In the larger tiers few cells are in flight and a launch lasts as long as
+// Few cells are in flight here and a launch lasts as long as
 // its longest cell, so what counts is the length of one wave's instruction
 // chain.  The longest cell of a 65 k point LiDAR scan (190 faces, 2800
 // candidates of which 440 cut) in tier 1, by cycle counts: of 15 M cycles
@@ -63,7 +56,6 @@ struct alignas(16) GroupLDS {
     float2 plx[P];
     uint32_t vtri[V];
     uint32_t tmp[P > 64 && P <= 256 && 2 * P > V ? 2 * P : V];  // (a 64-bit word per plane fits: clip())
-    uint32_t pm[P <= 64 ? (P + 1) / 2 : 1];
     uint32_t ctr[kNumCtr];  // diagnostics, in the order of the statistics slots
     uint32_t exact_events;  // removal tests of the current cell decided by expansion arithmetic
 };
@@ -339,7 +331,7 @@ __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirs
 __device__ __forceinline__ float uniform(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
 
 // ------------------------------------------------------------------ group
-template <int G, int V, int P, int L>
+template <int G, int V, int P>
 struct Group {
     static constexpr int kRows = V / G;               // vertex slots per lane
     static constexpr int kW = V / 64;                 // words of a vertex mask
@@ -348,12 +340,10 @@ struct Group {
     static constexpr uint64_t kRowMask = G == 64 ? ~0ull : ((1ull << G) - 1ull);
     static constexpr int kB = P < 256 ? 8 : 10;       // bits of a plane slot in a triple
     static constexpr uint32_t kBMask = (1u << kB) - 1u;
-    static_assert((G == 16 || G == 64) && L % kWave == 0 && V % 64 == 0 && P < (1 << kB) && 3 * kRows <= 64, "group geometry");
+    static_assert(G == 64 && V % 64 == 0 && P < (1 << kB) && 3 * kRows <= 64, "group geometry");
 
-    static constexpr int kLS = L / kWave;  // wait-list slots per lane
     GroupLDS<V, P> *S;
     CandLDS<G> *C;
-    uint32_t lr[kLS];
     uint32_t stk_node, stk_left;  // the wide walk's stack: entry t in lane t
     int gl;      // lane within the group
     int gshift;  // bit offset of the group in a wave ballot
@@ -802,8 +792,13 @@ struct Group {
             const uint32_t t0 = tri_get<kB>(tr, 0), t1 = tri_get<kB>(tr, 1), t2 = tri_get<kB>(tr, 2);
             bool tw0 = false, tw1 = false, tw2 = false;
             if constexpr (G == 64 && P <= 256) {
-                // As below, with 64-bit masks in tmp[] (each lane has read its
-                // triangle there), the words in use cleared first.
+                // The dual of a cell is a triangulated sphere: a pair of
+                // planes lies in at most two triangles, which then share it
+                // as an edge.  So the twin of edge (x, y) is removed iff
+                // another removed triangle holds both x and y: per plane, OR
+                // in the lanes whose removed triangle holds it intersect.  The
+                // words in use, in tmp[] (each lane has read its triangle
+                // there), are cleared first.
                 unsigned long long *pm = (unsigned long long *)S->tmp;
                 const unsigned long long bit = 1ull << gl;
                 if (has_tri) {
@@ -826,30 +821,6 @@ struct Group {
                     tw2 = (m2 & m0) != 0ull;
                 }
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            } else if constexpr (G == 16 && P <= 64) {
-                // The dual of a cell is a triangulated sphere: a pair of
-                // planes lies in at most two triangles, which then share it
-                // as an edge.  So the twin of edge (x, y) is removed iff
-                // another removed triangle holds both x and y: per plane, OR
-                // in the lanes whose removed triangle holds it (LDS
-                // operations of one wave complete in order), intersect, and
-                // clear the words again.
-                const uint32_t bit = 1u << gl;
-                if (has_tri) {
-                    atomicOr(&S->pm[t0 >> 1], bit << ((t0 & 1u) << 4));
-                    atomicOr(&S->pm[t1 >> 1], bit << ((t1 & 1u) << 4));
-                    atomicOr(&S->pm[t2 >> 1], bit << ((t2 & 1u) << 4));
-                    const uint32_t m0 = S->pm[t0 >> 1] >> ((t0 & 1u) << 4);
-                    const uint32_t m1 = S->pm[t1 >> 1] >> ((t1 & 1u) << 4);
-                    const uint32_t m2 = S->pm[t2 >> 1] >> ((t2 & 1u) << 4);
-                    const uint32_t others = 0xFFFFu & ~bit;
-                    tw0 = (m0 & m1 & others) != 0u;
-                    tw1 = (m1 & m2 & others) != 0u;
-                    tw2 = (m2 & m0 & others) != 0u;
-                    S->pm[t0 >> 1] = 0u;
-                    S->pm[t1 >> 1] = 0u;
-                    S->pm[t2 >> 1] = 0u;
-                }
             } else {
                 for (int u = 0; u < R; ++u) {  // broadcast reads of the removed triangles
                     const uint32_t o = S->tmp[u];
@@ -968,29 +939,11 @@ struct Group {
         return !too_far(c);
     }
 
-    // May the plane of the lane's own candidate cut the cell: is some vertex
-    // not certainly behind it (the test of beyond32, so a candidate refused
-    // here would be refused vertex by vertex in clip())?  The slots are read
-    // in order, each by the whole group at once; a free slot holds a radius
-    // that fails the test (retire_vertices).
-    __device__ __forceinline__ bool may_cut(const Cand &c) const {
-        const float c2 = fmaf(kG32, c.pH, kTiny32);
-        bool hit = false;
-#pragma unroll 1
-        for (int v = 0; v < V; v += 8) {
-            if (__ballot((valid[v >> 6] >> (v & 63)) != 0ull) == 0ull) break;
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const float4 p = S->vpos[v + u];
-                const float Pv = fmaf(c.ax, p.x, fmaf(c.ay, p.y, fmaf(c.az, p.z, -c.H)));
-                hit |= !(Pv < -fmaf(c.pa1, p.w, c2));
-            }
-        }
-        return hit;
-    }
-
-    // Those of the wave's candidates (todo) that may cut the cell, a candidate
-    // per lane as above; a leaf's (at most 32, in the low half) are copied to
+    // Those of the wave's candidates (todo) that may cut the cell: is some
+    // vertex not certainly behind the plane (the test of clip(), so a candidate
+    // refused here would be refused vertex by vertex there)?  A candidate per
+    // lane, the vertices in order (a free slot holds a record that fails the
+    // test: retire_vertices); a leaf's (at most 32, in the low half) are copied to
     // the high half, which takes every other vertex.
     __device__ __forceinline__ uint64_t may_cut_wave(const Cand &own_c, uint64_t todo) const {
         Cand c = own_c;
@@ -1020,7 +973,7 @@ struct Group {
         return todo & (halves ? hits | (hits >> 32) : hits);
     }
 
-    // Marks the slots of m as free for may_cut().
+    // Marks the slots of m as free for may_cut_wave().
     __device__ __forceinline__ void retire_vertices(const uint64_t (&m)[kW]) const {
 #pragma unroll
         for (int k = 0; k < kRows; ++k)
@@ -1047,8 +1000,7 @@ struct Group {
         // after this), so only the others are offered one at a time.
         // Nothing to gain on the initial box, which every guess cuts.
         if (np > 6 && todo) {
-            if constexpr (G == 16) todo = gballot(live_c && may_cut(c));
-            else todo = may_cut_wave(c, todo);
+            todo = may_cut_wave(c, todo);
             if (!todo) return;
         }
         if (live_c) {
@@ -1382,8 +1334,6 @@ struct Group {
         const int grp = lane / G;
         S = s;
         C = c;
-#pragma unroll
-        for (int j = 0; j < kLS; ++j) lr[j] = 0u;
         stk_node = stk_left = 0u;
         gl = lane & (G - 1);
         lane64 = lane;
@@ -1395,14 +1345,12 @@ struct Group {
         wide = prm.wide;
         if (prm.clouds == nullptr) set_cloud(prm.hdr, wide_ref((uint32_t)prm.n, 0u, (uint32_t)prm.n));
         if (gl < kNumCtr) S->ctr[gl] = 0u;
-        for (int w = gl; w < (int)(sizeof(S->pm) / 4); w += G) S->pm[w] = 0u;
     }
 
-    // The cloud the next cells belong to: its clipping box and subtree (the
-    // twin walks the binary form, the others the wide one).
+    // The cloud the next cells belong to: its clipping box and wide form.
     __device__ __forceinline__ void set_cloud(const IndexHeader *h, uint32_t wide_root) {
         hdr = h;
-        root_ref = G == 16 ? h->root_ref : wide_root;
+        root_ref = wide_root;
     }
     __device__ __forceinline__ void set_cloud(const CellParams &prm, int cl) {
         const int64_t a = prm.cloud_cells[cl], z = prm.cloud_cells[cl + 1];
@@ -1438,15 +1386,13 @@ __device__ __forceinline__ int batch_find(const int64_t *off, int n_clouds, int6
 }
 
 // ------------------------------------------------------------------ tiers
-constexpr int kT0Lanes = 16, kT0Verts = 64, kT0Planes = 48, kT0List = 128, kT0Threads = 256;
-// (a depth-first stack holds at most one entry per level of the hierarchy,
-// fewer than 64 levels: 128 entries never fill)
-constexpr int kTmLanes = 64, kTmVerts = 192, kTmPlanes = 128, kTmList = 128, kTmThreads = 128;
-constexpr int kT1Lanes = 64, kT1Verts = 512, kT1Planes = 255, kT1List = 128, kT1Threads = 128;
-constexpr int kT2Lanes = 64, kT2Verts = 1024, kT2Planes = 1023, kT2List = 128, kT2Threads = 64;
-using TierM = Group<kTmLanes, kTmVerts, kTmPlanes, kTmList>;
-using Tier1 = Group<kT1Lanes, kT1Verts, kT1Planes, kT1List>;
-using Tier2 = Group<kT2Lanes, kT2Verts, kT2Planes, kT2List>;
+constexpr int kT0Lanes = 16, kT0Verts = 64, kT0Planes = 48, kT0Threads = 256;
+constexpr int kTmLanes = 64, kTmVerts = 192, kTmPlanes = 128, kTmThreads = 128;
+constexpr int kT1Lanes = 64, kT1Verts = 512, kT1Planes = 255, kT1Threads = 128;
+constexpr int kT2Lanes = 64, kT2Verts = 1024, kT2Planes = 1023, kT2Threads = 64;
+using TierM = Group<kTmLanes, kTmVerts, kTmPlanes>;
+using Tier1 = Group<kT1Lanes, kT1Verts, kT1Planes>;
+using Tier2 = Group<kT2Lanes, kT2Verts, kT2Planes>;
 
 // The address of the block's copy of the launch's parameters (in LDS: one
 // copy per block, where a kernel argument whose address is taken would be
@@ -1512,10 +1458,10 @@ __global__ void __launch_bounds__(256) cell_flagged_kernel(const CellParams prm)
 
 // Decides in FP64 (where FP64 cannot, exactly) the removal tests tier 0 took
 // by their FP32 sign, and flags the cell of every test whose sign was wrong
-// for the FP64-capable twin, which rebuilds the cell (its row, count and
+// for tier m, which rebuilds the cell (its row, count and
 // status replace tier 0's).  A test whose vertex lies on a plane of a
 // predicted cube (owner codes -7..-12, not a plane of the diagram) is not
-// decided: its cell is flagged as well, and the twin builds it without the
+// decided: its cell is flagged as well, and tier m builds it without the
 // cube.  One thread per recorded test.
 __global__ void __launch_bounds__(256) cell_tentative_check_kernel(const CellParams prm) {
     const uint32_t m = min(prm.counters[7], prm.tent_cap);
@@ -1619,7 +1565,7 @@ __device__ __forceinline__ void queued_tier_body(const CellParams &prm, const ui
 }
 
 // Tier m: 192 vertices / 128 planes at three waves per SIMD, the cells tier 0
-// (or its twin) gave up on capacity.
+// gave up on capacity, and the flagged ones.
 __global__ void __launch_bounds__(kTmThreads) __attribute__((amdgpu_waves_per_eu(3, 3)))
 cell_group_mid_kernel(const CellParams prm) {
     queued_tier_body<TierM, kTmVerts, kTmPlanes, kTmThreads, 1, 8, true>(prm, prm.mid_list, prm.big_list);
