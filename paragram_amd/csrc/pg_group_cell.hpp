@@ -319,6 +319,11 @@ __device__ __forceinline__ float rl(float x, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
 }
 
+// Orders the wave's accesses to LDS for the compiler, which keeps a store of
+// one lane and a load of the same word by another in program order only across
+// a fence.  It is no instruction: the LDS operations of a wave complete in order.
+__device__ __forceinline__ void lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local"); }
+
 // A word that other lanes of the wave have written.
 __device__ __forceinline__ unsigned long long lds_load(const unsigned long long *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);

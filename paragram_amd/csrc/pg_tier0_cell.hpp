@@ -345,6 +345,7 @@ struct Tier0 {
             }
             // every lane has read slot p before any lane writes a slot below
             // G (k + 1): all later reads are at or above that
+            lds_fence();
             if (mv) {
                 const int dst = __popcll(used & ((1ull << p) - 1ull));
                 S->pl[dst] = a;
@@ -355,6 +356,7 @@ struct Tier0 {
         for (int k = 0; k < kRows; ++k)
             if (gl + G * k < nv) S->vtri[gl + G * k] = renumber(used, S->vtri[gl + G * k]);
         if ((uint32_t)gl < nt) S->tent[gl][0] = renumber(used, S->tent[gl][0]);
+        lds_fence();
         np = __popcll(used);
     }
 
@@ -430,6 +432,7 @@ struct Tier0 {
                 }
             }
             S->ntent = n0 + (uint32_t)tot;
+            lds_fence();
         }
         const int R = __popc(rem0) + __popc(rem1);
         if (R == 0) return false;  // the plane does not cut
@@ -449,6 +452,7 @@ struct Tier0 {
             return true;
         }
         if (np >= P) {
+            lds_fence();  // (the list; a lane stores to entries that others wrote)
             garbage_collect();
             if (np >= P) {
                 overflow = true;
@@ -467,6 +471,7 @@ struct Tier0 {
             S->pl[qs] = q;
             S->own[qs] = owner;
         }
+        lds_fence();  // the list and the new plane
         if (in_guess) bloom |= bloom_bit((uint32_t)owner);
         // Boundary of the removed triangles: directed edges whose twin is not
         // removed.  Its nb edges are compacted into tmp[0, nb).
@@ -490,21 +495,26 @@ struct Tier0 {
             // lies in at most two triangles, which then share it as an edge.
             // So the twin of edge (x, y) is removed iff another removed
             // triangle holds both x and y: per plane, OR in the lanes whose
-            // removed triangle holds it (LDS operations of one wave complete
-            // in order), intersect, and clear the words again.
+            // removed triangle holds it, intersect, and clear the words again.
             {
                 const uint32_t bit = 1u << gl;
+                const uint32_t s0 = (t0 & 1u) << 4, s1 = (t1 & 1u) << 4, s2 = (t2 & 1u) << 4;
+                uint32_t *w0 = &S->pm[t0 >> 1], *w1 = &S->pm[t1 >> 1], *w2 = &S->pm[t2 >> 1];
                 if (has_tri) {
-                    const uint32_t s0 = (t0 & 1u) << 4, s1 = (t1 & 1u) << 4, s2 = (t2 & 1u) << 4;
-                    uint32_t *w0 = &S->pm[t0 >> 1], *w1 = &S->pm[t1 >> 1], *w2 = &S->pm[t2 >> 1];
                     atomicOr(w0, bit << s0);
                     atomicOr(w1, bit << s1);
                     atomicOr(w2, bit << s2);
+                }
+                lds_fence();
+                if (has_tri) {
                     const uint32_t m0 = *w0 >> s0, m1 = *w1 >> s1, m2 = *w2 >> s2;
                     const uint32_t others = 0xFFFFu & ~bit;
                     tw0 = (m0 & m1 & others) != 0u;
                     tw1 = (m1 & m2 & others) != 0u;
                     tw2 = (m2 & m0 & others) != 0u;
+                }
+                lds_fence();
+                if (has_tri) {
                     *w0 = 0u;
                     *w1 = 0u;
                     *w2 = 0u;
@@ -526,6 +536,7 @@ struct Tier0 {
             // in its word
             uint32_t emask = 0;
             boundary_rows(rem0, rem1, R, emask, cycle);
+            lds_fence();  // (every lane has read the list)
             int j = gexcl(__popc(emask), nb);
             // (a removed set of R triangles without gaps has at most R + 2
             // boundary edges; more than tmp holds are never written)
@@ -549,6 +560,7 @@ struct Tier0 {
             overflow = true;
             return false;
         }
+        lds_fence();  // the edges
         // One new vertex (q, x, y) per boundary edge: the first R take the
         // removed ones' slots, the others follow the last vertex.
         bool bad = false;
@@ -561,6 +573,7 @@ struct Tier0 {
             // fewer new than removed: the last vertices move into the slots
             // left over (those of the removed list from nb on, in order)
             if (spread && gl >= nb && gl < R) S->tmp[gl] = my_slot;
+            lds_fence();
             int m = nb;
 #pragma unroll
             for (int k = 0; k < kRows; ++k) {
@@ -577,6 +590,7 @@ struct Tier0 {
                 m += __popc(bits);
             }
         }
+        lds_fence();  // the vertices
         nv = kept + nb;
         if (gany(bad)) {
             overflow = true;
@@ -674,7 +688,8 @@ struct Tier0 {
         // after this), so only the others are offered one at a time.
         // Nothing to gain on the initial box, which every guess cuts.
         if (np > 6) {
-            live_c = live_c && may_cut(c);
+            const bool cuts = may_cut(c);  // (by all lanes of the group)
+            live_c = live_c && cuts;
             todo = gballot(live_c);
             if (!todo) return false;
         }
@@ -683,6 +698,7 @@ struct Tier0 {
             S->cand[gl] = c;
             S->cown[gl] = (int)(maybe_guess ? (j | 0x80000000u) : j);
         }
+        lds_fence();
         float hkey = live_c ? c.w : FLT_MAX;
         while (todo) {
             // nearest plane first (smallest H = power distance of the point):
@@ -703,6 +719,7 @@ struct Tier0 {
                 return true;
             }
         }
+        lds_fence();  // (the next batch is staged in the same place)
         if (!dirty) return false;
         update_bounds();
         dirty = false;
@@ -737,6 +754,7 @@ struct Tier0 {
             S->pl[gl] = pl;
             S->own[gl] = (from_cube ? -7 : -1) - gl;
         }
+        lds_fence();
         cube = gany(from_cube);
         np = 6;
         nv = 8;
@@ -749,6 +767,7 @@ struct Tier0 {
             if (sgn > 0) make_vertex(gl, X, Y, Z);
             else make_vertex(gl, X, Z, Y);
         }
+        lds_fence();
         bloom = 0;
         update_bounds();
         dirty = false;
@@ -999,6 +1018,7 @@ struct Tier0 {
 #pragma unroll
         for (int k = 0; k < kPRows; ++k)
             if (ids[k] >= 0) S->tmp[at++] = (uint32_t)ids[k];
+        lds_fence();
         return F;
     }
 
