@@ -706,6 +706,7 @@ struct Group {
             }
             // every lane has read slot p before any lane writes a slot below
             // G (k + 1): all later reads are at or above that
+            lds_fence();
             if (mv) {
                 const uint32_t dst = plane_rank(used, (uint32_t)p);
                 S->pl[dst] = a;
@@ -721,6 +722,7 @@ struct Group {
                                          plane_rank(used, tri_get<kB>(t, 2)));
             }
         }
+        lds_fence();
         np = mask_popc(used);
     }
 
@@ -774,6 +776,7 @@ struct Group {
             S->pl[qs] = make_float4(q.ax, q.ay, q.az, q.H);
             S->plx[qs] = make_float2(q.pH, __int_as_float(q.owner));
         }
+        lds_fence();
         if (in_guess) bloom |= bloom_bit((uint32_t)q.owner);
         // Boundary of the removed triangles: directed edges whose twin is not
         // removed; bit 3r + e of emask marks edge e of the lane's r-th
@@ -792,6 +795,7 @@ struct Group {
                 if ((bits >> gl) & 1ull) S->tmp[base + __popcll(bits & ((1ull << gl) - 1ull))] = S->vtri[gl + G * k];
                 base += __popcll(bits);
             }
+            lds_fence();
             const bool has_tri = gl < R;
             tr = has_tri ? S->tmp[gl] : 0u;
             const uint32_t t0 = tri_get<kB>(tr, 0), t1 = tri_get<kB>(tr, 1), t2 = tri_get<kB>(tr, 2);
@@ -806,18 +810,19 @@ struct Group {
                 // there), are cleared first.
                 unsigned long long *pm = (unsigned long long *)S->tmp;
                 const unsigned long long bit = 1ull << gl;
+                lds_fence();
                 if (has_tri) {
                     pm[t0] = 0ull;
                     pm[t1] = 0ull;
                     pm[t2] = 0ull;
                 }
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                lds_fence();
                 if (has_tri) {
                     atomicOr(&pm[t0], bit);
                     atomicOr(&pm[t1], bit);
                     atomicOr(&pm[t2], bit);
                 }
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                lds_fence();
                 if (has_tri) {
                     const unsigned long long m0 = lds_load(&pm[t0]) & ~bit, m1 = lds_load(&pm[t1]) & ~bit,
                                              m2 = lds_load(&pm[t2]) & ~bit;
@@ -825,7 +830,7 @@ struct Group {
                     tw1 = (m1 & m2) != 0ull;
                     tw2 = (m2 & m0) != 0ull;
                 }
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                lds_fence();
             } else {
                 for (int u = 0; u < R; ++u) {  // broadcast reads of the removed triangles
                     const uint32_t o = S->tmp[u];
@@ -833,6 +838,7 @@ struct Group {
                     tw1 |= tri_has_edge<kB>(o, t2, t1);
                     tw2 |= tri_has_edge<kB>(o, t0, t2);
                 }
+                lds_fence();
             }
 #pragma unroll
             for (int e = 0; e < 3; ++e) {
@@ -871,6 +877,7 @@ struct Group {
             const uint32_t t = spread ? tr : S->vtri[gl + G * k];
             S->tmp[j++] = tri_get<kB>(t, e) | (tri_get<kB>(t, e == 2 ? 0 : e + 1) << kB);
         }
+        lds_fence();
         // one new vertex (q, x, y) per boundary edge, in the free slots
         // (lowest first), lane-strided
         bool bad = false;
@@ -880,11 +887,13 @@ struct Group {
         }
         uint64_t added[kW];
         mask_first(freem, nb, added);
+        lds_fence();
         if (gany(bad)) fix_vertices(added);
         uint64_t freed[kW];
 #pragma unroll
         for (int w = 0; w < kW; ++w) freed[w] = rem[w] & ~added[w];
         retire_vertices(freed);
+        lds_fence();
 #pragma unroll
         for (int w = 0; w < kW; ++w) valid[w] = (valid[w] & ~rem[w]) | added[w];
         dirty = true;
@@ -1013,6 +1022,7 @@ struct Group {
             // the owner's sign bit marks a candidate that may already own a plane
             C->po[gl] = make_float2(c.pH, __int_as_float(maybe_guess ? (c.owner | INT32_MIN) : c.owner));
         }
+        lds_fence();
         float hkey = live_c ? c.H : FLT_MAX;
         while (todo) {
             // nearest plane first (smallest H = power distance of the point):
@@ -1042,6 +1052,7 @@ struct Group {
                 return;
             }
         }
+        lds_fence();  // (the next batch is staged in the same place)
         if (dirty) {
             update_bounds();
             dirty = false;
@@ -1066,6 +1077,7 @@ struct Group {
             S->plx[gl] = make_float2(fabsf(h), __int_as_float(-1 - gl));
         }
         np = 6;
+        lds_fence();
         // the 8 corners go to slots 0..7 (lanes 0..7 of row 0)
         if (gl < 8) {
             const int cx = gl >> 2 & 1, cy = gl >> 1 & 1, cz = gl & 1;
@@ -1082,6 +1094,7 @@ struct Group {
             unused[w] = ~valid[w];
         }
         retire_vertices(unused);
+        lds_fence();
         bloom = 0;
         update_bounds();
         dirty = false;
@@ -1210,6 +1223,7 @@ struct Group {
 #pragma unroll
         for (int k = 0; k < kPRows; ++k)
             if (ids[k] >= 0) S->tmp[at++] = (uint32_t)ids[k];
+        lds_fence();
         return F;
     }
 
@@ -1363,6 +1377,7 @@ struct Group {
     }
 
     __device__ __forceinline__ void flush(const CellParams &prm, uint32_t cells) const {
+        lds_fence();
         uint32_t vals[kNumCtr];
 #pragma unroll
         for (int k = 0; k < kNumCtr; ++k) vals[k] = gl == 0 ? S->ctr[k] : 0u;
@@ -1542,6 +1557,7 @@ __device__ __forceinline__ void queued_tier_body(const CellParams &prm, const ui
             if (k < prm.promo_cap) g.offer_owners(prm.promo + (size_t)k * kPromoPlanes, kPromoPlanes);
         }
         g.traverse();
+        lds_fence();  // (the lanes' counts)
         const CellParams &Q = *reread(&sprm);
         const uint32_t orig = Q.perm[cell];
         if (lane == 0 && g.S->exact_events) log_exact(Q, orig, g.S->exact_events);
@@ -1605,6 +1621,7 @@ __global__ void __launch_bounds__(kT2Threads) cell_group_huge_kernel(const CellP
         g.active = true;
         g.start(cell, *reread(&sprm));
         g.traverse();
+        lds_fence();  // (the lanes' counts)
         const CellParams &P = *reread(&sprm);
         const uint32_t orig = P.perm[cell];
         if (lane == 0 && g.S->exact_events) log_exact(P, orig, g.S->exact_events);

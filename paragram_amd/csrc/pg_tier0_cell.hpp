@@ -1115,6 +1115,7 @@ struct Tier0 {
 
     // Adds the wave's counters to the launch's (cells: every lane's count).
     __device__ __forceinline__ void flush(const CellParams &prm, uint32_t cells) const {
+        lds_fence();
         const uint32_t total = wave_sum(cells);
         if (lane64 < kNumCtr) {
             const uint32_t s = lane64 == kStatCells ? total : ctr[lane64];

@@ -144,6 +144,7 @@ struct Larger {
         T g;
         g.setup(prm, &both.lds, &both.cand);
         g.set_cloud(&hdr, root);
+        emu::fence();
         for (int32_t cell : cells) {
             g.active = true;
             const uint32_t before = g.gl == 0 ? both.lds.ctr[kStatClips] : 0u;

@@ -85,3 +85,12 @@ def test_tier_0(prog, name, walk):
         assert got.kept.mean() > 0.9 and (got.open_tests == 0).mean() > 0.5
     if name == "hub_160":
         assert not got.kept[0], "a cell of 160 faces in 48 plane slots"
+
+
+@pytest.mark.parametrize("walk", list(WALKS))
+@pytest.mark.parametrize("name", ["clamped", "hub_40", "hub_160", "chain", "grid_8"])
+@pytest.mark.parametrize("tier", ["m", "1", "2"])
+def test_larger_tiers(prog, tier, name, walk):
+    got = check(prog, name, tier, walk, 12)
+    if name == "hub_160":  # in 128, 255 and 1023 plane slots
+        assert bool(got.kept[0]) == (tier != "m")
