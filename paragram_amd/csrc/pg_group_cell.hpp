@@ -1017,18 +1017,19 @@ struct Group {
             todo = may_cut_wave(c, todo);
             if (!todo) return;
         }
-        if (live_c) {
+        const bool in = ((todo >> gl) & 1ull) != 0ull;  // (the lanes that the test above dropped take no further part)
+        if (in) {
             C->aH[gl] = make_float4(c.ax, c.ay, c.az, c.H);
             // the owner's sign bit marks a candidate that may already own a plane
             C->po[gl] = make_float2(c.pH, __int_as_float(maybe_guess ? (c.owner | INT32_MIN) : c.owner));
         }
         lds_fence();
-        float hkey = live_c ? c.H : FLT_MAX;
+        float hkey = in ? c.H : FLT_MAX;
         while (todo) {
             // nearest plane first (smallest H = power distance of the point):
             // the cell shrinks fastest and fewer clips are undone later
             const float hmin = gmin(hkey);
-            const uint64_t at = gballot(live_c && hkey == hmin) & todo;
+            const uint64_t at = gballot(hkey == hmin) & todo;
             const int b = (int)__builtin_ctzll(at ? at : todo);
             todo &= ~(1ull << b);
             if (gl == b) hkey = FLT_MAX;

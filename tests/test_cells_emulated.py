@@ -94,3 +94,28 @@ def test_larger_tiers(prog, tier, name, walk):
     got = check(prog, name, tier, walk, 12)
     if name == "hub_160":  # in 128, 255 and 1023 plane slots
         assert bool(got.kept[0]) == (tier != "m")
+
+
+@pytest.mark.parametrize("tier", ["0", "m", "1", "2"])
+def test_a_batch_is_offered_nearest_first(prog, tier):
+    """The candidates of a leaf that may cut are clipped in the order of their
+    distance, whatever their places in it and whichever of the others the test
+    against the vertices has dropped: the planes held past the guesses' stand in
+    that order."""
+    leaf = 16 if tier == "0" else 32  # points of one batch
+    held = 0
+    for seed in range(12):
+        r = np.random.default_rng(seed)
+        pts = r.random((leaf, 3)).astype(np.float32)
+        pts[r.permutation(leaf)[: leaf // 2]] += 2.0  # far ones, which the filter drops
+        order = r.permutation(leaf)
+        guesses = np.stack([r.permutation(leaf)[:6] for _ in range(leaf)])
+        got = emu.run(prog, pts, tier=tier, order=order, guesses=guesses)
+        inv = np.argsort(order)
+        for k in range(leaf):
+            first = set(order[guesses[inv[k]]].tolist())
+            later = [o for o in got.held[k].tolist() if o >= 0 and o not in first]
+            d = ((pts[later] - pts[k]).astype(np.float64) ** 2).sum(1)
+            assert (np.diff(d) > 0).all(), f"seed {seed}, cell {k}"
+            held += len(later)
+    assert held > 100
