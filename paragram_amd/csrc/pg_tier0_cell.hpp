@@ -1254,7 +1254,7 @@ __device__ __forceinline__ void tier0_body(const CellParams &prm) {
             if (slot < P.promo_cap) g.store_owners(P.promo + (size_t)slot * kPromoPlanes);
         }
         if (active && P.cycles && g.gl == 0) P.cycles[orig] = (uint32_t)min(clock64() - t0, (uint64_t)0x7fffffff);
-        if (active && g.gl == 0 && !g.bail) cells++;
+        if (active && g.gl == 0) cells++;
     }
     g.flush(prm, cells);
 }
