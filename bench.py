@@ -51,19 +51,21 @@ WORKLOADS = {
            "{total:,} points in all), seed {seed}, one launch"),
 }
 TRAFFIC_PATH = os.path.join(ROOT, "profiles", "cell_kernel_traffic.json")
-CELL_KERNELS = ("cell_group_kernel", "cell_tentative_check_kernel", "cell_flagged_kernel",
+TIER0_KERNELS = ("cell_group_kernel", "cell_group_small_kernel")  # one of them per launch
+CELL_KERNELS = (*TIER0_KERNELS, "cell_tentative_check_kernel", "cell_flagged_kernel",
                 "cell_group_mid_kernel", "cell_group_big_kernel", "cell_group_huge_kernel")
 COPY_KERNEL = "__amd_rocclr_copyBuffer"
 
 
 def _traffic_record(workload_key: str):
-    """HBM bytes per cell-construction launch from the committed rocprofv3 PMC summary, if any."""
+    """HBM bytes per cell-construction launch from the committed rocprofv3 PMC summary, if there
+    is one of the kernels that run now."""
     try:
         with open(TRAFFIC_PATH) as f:
-            rec = json.load(f)
-        return rec.get(workload_key)
+            rec = json.load(f).get(workload_key)
     except (OSError, ValueError):
         return None
+    return rec if rec and rec.get("kernels") == list(CELL_KERNELS) else None
 
 
 def _pmc_values(run_dir: str, counter: str):
@@ -95,7 +97,7 @@ def summarize_pmc(fetch_dir: str, write_dir: str, copy_mib: int, workload_key: s
             short = name.split("(")[0].split("::")[-1]
             if short in CELL_KERNELS:
                 per_kernel.setdefault(short, []).append(v)
-        launches = len(per_kernel.get(CELL_KERNELS[0], []))
+        launches = sum(len(per_kernel.get(k, [])) for k in TIER0_KERNELS)
         kib = sum(sum(v) for v in per_kernel.values()) / max(launches, 1)
         res[counter] = {"kib_per_launch_raw": round(kib, 1), "copy_factor": round(factor, 4),
                         "bytes_per_launch": round(kib * 1024.0 / factor)}
