@@ -700,6 +700,7 @@ static hipError_t build_tail(int64_t n, const float *points, const float *weight
             hipLaunchKernelGGL(refit_top_kernel, dim3(grid_for(n - 1, 256)), dim3(256), 0, stream, sorted, n, children,
                                parents, ranges, boxes, flags, nodes, leaf_size);
         // the wide form takes the boxes' place
+        if (!wide_fits((uint32_t)n)) return hipErrorInvalidValue;
         if (n > kWideLeaf)
             hipLaunchKernelGGL(wide_kernel, dim3(grid_for(n - 1, 256)), dim3(256), 0, stream, nodes, n, parents, ranges,
                                keys, 32 - cloud_bits, (WideChild *)boxes);

@@ -10,9 +10,9 @@
 //
 // Wide nodes need no allocation: subtrees of one class are disjoint ranges of
 // at least L = 32 * 8^(k-1) + 1 points, so first / L numbers them without
-// collision.  All classes together take less than n / 28 records of 512
-// bytes, less than the 32 bytes per point that the refit's boxes occupy, and
-// live there once the refit has read them.
+// collision.  The records of all classes (512 bytes each; for large n one per
+// 28 points) fit into the 32 bytes per binary node of the refit's boxes at
+// every n (wide_fits), and live there once the refit has read them.
 #pragma once
 
 #include "pg_common.hpp"
@@ -51,6 +51,10 @@ __host__ __device__ inline uint64_t wide_records(uint32_t n) {
     uint64_t r = 0;
     for (int k = 1; k <= wide_class(n); ++k) r += (n - 1u) / wide_least(k) + 1u;
     return r;
+}
+// do they fit into the boxes of the n - 1 binary nodes?
+__host__ __device__ inline bool wide_fits(uint32_t n) {
+    return n <= (uint32_t)kWideLeaf || 16ull * sizeof(WideChild) * wide_records(n) <= 32ull * (n - 1u);
 }
 
 }  // namespace pg
