@@ -1,6 +1,8 @@
 """Autotuner for the launch choices that change speed but never the diagram:
 the LBVH leaf size, the number of nearest neighbours clipped first, and the
-persistent waves per compute unit of the cell launch.
+persistent waves per compute unit of the cell launch.  The cells walk 32-point
+leaves whatever the leaf size; it is read by the nearest-neighbour search of
+calls of more than 196608 points, and only there is it tuned.
 
 ``tune(points, weights)`` times every candidate on a bounded prefix of the
 caller's own data (2 calls each after one warm-up) and returns the fastest;
@@ -25,6 +27,7 @@ import torch
 from . import _api, _engine
 
 LEAF_SIZES = (8, 16, 32)
+LEAF_FREE = 3 << 16  # up to this many points nothing on the way to the diagram reads the leaf size
 PRECLIPS = (8, 16)
 WAVES_PER_CU = (12, 16, 24)  # 12 = what tier 0 keeps resident (3 per SIMD); more queue behind them
 SAMPLE = 200_000
@@ -52,8 +55,8 @@ def _save_file():
 def tune(points: torch.Tensor, weights: torch.Tensor | None = None, clouds=None, sample: int = SAMPLE,
          force: bool = False) -> dict:
     """The fastest {leaf_size, preclip, waves_per_cu} for data like ``points`` (timed on up to
-    ``sample`` of them): leaf size and pre-clip over their grid at the default waves, then the
-    waves per compute unit at the best of those."""
+    ``sample`` of them): leaf size and pre-clip over their grid at the default waves (the
+    leaf size where it matters), then the waves per compute unit at the best of those."""
     from ._backend import _C
 
     n = int(points.shape[0])
@@ -86,7 +89,7 @@ def tune(points: torch.Tensor, weights: torch.Tensor | None = None, clouds=None,
         times[f"{cfg['leaf_size']}/{cfg['preclip']}/{cfg['waves_per_cu']}"] = round(t * 1e3, 3)
         return t
 
-    for leaf in LEAF_SIZES:
+    for leaf in LEAF_SIZES if m > LEAF_FREE else LEAF_SIZES[-1:]:
         for pre in PRECLIPS:
             cfg = {"leaf_size": leaf, "preclip": pre, "waves_per_cu": 16}
             t = timed(cfg)
