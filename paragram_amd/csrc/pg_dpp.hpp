@@ -18,10 +18,6 @@ template <int C>
 __device__ __forceinline__ int dpp(int x) {
     return __builtin_amdgcn_update_dpp(0, x, C, 0xF, 0xF, true);  // lanes shifted in from outside the row read 0
 }
-template <int C>
-__device__ __forceinline__ float dppf(float x) {
-    return __int_as_float(dpp<C>(__float_as_int(x)));
-}
 // Float minima and maxima over a row through an order-preserving integer
 // key (sign-magnitude bits turned into two's complement): each step is one
 // integer min or max with the DPP operand folded in, where fminf/fmaxf of a

@@ -342,7 +342,6 @@ struct Group {
     static constexpr int kW = V / 64;                 // words of a vertex mask
     static constexpr int kPW = (P + 63) / 64;         // words of a plane mask
     static constexpr int kPRows = (P + G - 1) / G;    // plane slots per lane
-    static constexpr uint64_t kRowMask = G == 64 ? ~0ull : ((1ull << G) - 1ull);
     static constexpr int kB = P < 256 ? 8 : 10;       // bits of a plane slot in a triple
     static constexpr uint32_t kBMask = (1u << kB) - 1u;
     static_assert(G == 64 && V % 64 == 0 && P < (1 << kB) && 3 * kRows <= 64, "group geometry");
@@ -351,7 +350,6 @@ struct Group {
     CandLDS<G> *C;
     uint32_t stk_node, stk_left;  // the wide walk's stack: entry t in lane t
     int gl;      // lane within the group
-    int gshift;  // bit offset of the group in a wave ballot
     int lane64;
 
     const float4 *pts;
@@ -385,51 +383,41 @@ struct Group {
     __device__ __forceinline__ void count(int slot, uint32_t v = 1u) const { atomicAdd(&S->ctr[slot], v); }
 
     // ---------------------------------------------------------- group ops
-    __device__ __forceinline__ uint64_t gballot(bool p) const { return (__ballot(p) >> gshift) & kRowMask; }
+    __device__ __forceinline__ uint64_t gballot(bool p) const { return __ballot(p); }
     __device__ __forceinline__ bool gany(bool p) const { return gballot(p) != 0ull; }
     __device__ __forceinline__ bool live() const { return active && status == kSuccess && !overflow; }
     __device__ __forceinline__ int gbi(int x, int k) const { return __shfl(x, k, G); }
     // Reductions and scans: DPP within each 16-lane row, rows combined
-    // through readlane when the group is the whole wave.
+    // through readlane.
     __device__ __forceinline__ uint64_t gor64(uint64_t x) const {
         uint32_t lo = row_or((uint32_t)x), hi = row_or((uint32_t)(x >> 32));
-        if constexpr (G == 64) {
-            lo = rl(lo, 0) | rl(lo, 16) | rl(lo, 32) | rl(lo, 48);
-            hi = rl(hi, 0) | rl(hi, 16) | rl(hi, 32) | rl(hi, 48);
-        }
+        lo = rl(lo, 0) | rl(lo, 16) | rl(lo, 32) | rl(lo, 48);
+        hi = rl(hi, 0) | rl(hi, 16) | rl(hi, 32) | rl(hi, 48);
         return ((uint64_t)hi << 32) | lo;
     }
     __device__ __forceinline__ float gmin(float x) const {
         x = row_min(x);
-        if constexpr (G == 64) x = fminf(fminf(rl(x, 0), rl(x, 16)), fminf(rl(x, 32), rl(x, 48)));
-        return x;
+        return fminf(fminf(rl(x, 0), rl(x, 16)), fminf(rl(x, 32), rl(x, 48)));
     }
     __device__ __forceinline__ float gmax(float x) const {
         x = row_max(x);
-        if constexpr (G == 64) x = fmaxf(fmaxf(rl(x, 0), rl(x, 16)), fmaxf(rl(x, 32), rl(x, 48)));
-        return x;
+        return fmaxf(fmaxf(rl(x, 0), rl(x, 16)), fmaxf(rl(x, 32), rl(x, 48)));
     }
     __device__ __forceinline__ int gsum(int x) const {
         x = row_sum(x);
-        if constexpr (G == 64) x = rl(x, 0) + rl(x, 16) + rl(x, 32) + rl(x, 48);
-        return x;
+        return rl(x, 0) + rl(x, 16) + rl(x, 32) + rl(x, 48);
     }
     // exclusive prefix sum over the group; total in `tot`
     __device__ __forceinline__ int gexcl(int x, int &tot) const {
         const int incl = row_scan(x);
-        if constexpr (G == 16) {
-            tot = row_sum(x);
-            return incl - x;
-        } else {
-            const int t0 = rl(incl, 15), t1 = rl(incl, 31), t2 = rl(incl, 47), t3 = rl(incl, 63);
-            const int r = lane64 >> 4;
-            tot = t0 + t1 + t2 + t3;
-            return incl - x + (r > 0 ? t0 : 0) + (r > 1 ? t1 : 0) + (r > 2 ? t2 : 0);
-        }
+        const int t0 = rl(incl, 15), t1 = rl(incl, 31), t2 = rl(incl, 47), t3 = rl(incl, 63);
+        const int r = lane64 >> 4;
+        tot = t0 + t1 + t2 + t3;
+        return incl - x + (r > 0 ? t0 : 0) + (r > 1 ? t1 : 0) + (r > 2 ? t2 : 0);
     }
     // row k of a vertex mask: the bits of slots gl + G k, lane order
     __device__ __forceinline__ uint64_t row(const uint64_t (&m)[kW], int k) const {
-        return (m[(G * k) >> 6] >> ((G * k) & 63)) & kRowMask;
+        return m[(G * k) >> 6];
     }
     __device__ __forceinline__ bool own(const uint64_t (&m)[kW], int k) const {
         return (row(m, k) >> gl) & 1ull;
@@ -587,11 +575,10 @@ struct Group {
     //    the box overlaps, so no cut when |a|^2 - rho |a| - dw >= 0 for all
     //    |a| >= d, i.e. 2d >= rho and (d^2 - dw)^2 >= rho^2 d^2, d^2 > dw;
     //  * the per-vertex balls (balls_clear), the exact form.
-    // kSplit: the two halves of the group test two boxes at once (each lane
-    // is given its half's box).  kOctants: the first test alone, each lane its
-    // own box; kBalls: the second alone.
-    enum NodeTest { kBoth, kOctants, kBalls };
-    template <bool kSplit, NodeTest kTest = kBoth>
+    // kOctants: the first test, each lane its own box; kBalls: the second, one
+    // box by the whole wave.
+    enum NodeTest { kOctants, kBalls };
+    template <NodeTest kTest>
     __device__ __forceinline__ bool node_prunable(float4 lo, float4 hi, float &key) const {
         const float alx = lo.x - sx, aly = lo.y - sy, alz = lo.z - sz;
         const float ahx = hi.x - sx, ahy = hi.y - sy, ahz = hi.z - sz;
@@ -603,9 +590,9 @@ struct Group {
         const float hlow = d2 - dw;
         key = hlow;
         const float wslack = kSlack * (fabsf(lo.w) + fabsf(sw)) + kTiny32;
-        if constexpr (kTest == kBalls) return bounded && balls_clear<kSplit>(alx, aly, alz, ahx, ahy, ahz, dw + wslack);
-        // a box that holds the seed meets every vertex's ball (each passes
-        // through the seed), so neither test below can prune it
+        if constexpr (kTest == kBalls) return bounded && balls_clear(alx, aly, alz, ahx, ahy, ahz, dw + wslack);
+        // (a box that holds the seed meets every vertex's ball, as each passes
+        // through the seed)
         if (!bounded || d2 == 0.0f) return false;
         // the octants a box overlaps form a product set, so the largest
         // corner radius over them is a sum of per-axis maxima
@@ -615,9 +602,7 @@ struct Group {
                            (1.0f + kSlack);
         const float d2lo = d2 * (1.0f - kSlack);
         const float h = d2lo - dw - wslack;
-        if (4.0f * d2lo > rho2 && h > 0.0f && h * h > rho2 * d2 * (1.0f + kSlack)) return true;
-        if constexpr (kTest == kOctants) return false;
-        return balls_clear<kSplit>(alx, aly, alz, ahx, ahy, ahz, dw + wslack);
+        return 4.0f * d2lo > rho2 && h > 0.0f && h * h > rho2 * d2 * (1.0f + kSlack);
     }
 
     // Exact form of the prune, per vertex.  Vertex y is beyond the plane of
@@ -626,23 +611,18 @@ struct Group {
     // the seed (grown by the weight difference).  No point of the box cuts the
     // cell when the box misses every vertex's ball.  The box [2 al, 2 ah] is
     // widened by the cell's largest error radius (each coordinate of y lies
-    // within w of y~), and sum_k (|y~_k| + w)^2 bounds |y|^2.  The lanes that
-    // test one box (the group, or its half when kSplit) share the vertex
-    // slots.
-    template <bool kSplit>
+    // within w of y~), and sum_k (|y~_k| + w)^2 bounds |y|^2.  The wave's
+    // lanes share the vertex slots.
     __device__ __forceinline__ bool balls_clear(float alx, float aly, float alz, float ahx, float ahy, float ahz,
                                                 float dwmax) const {
-        constexpr int H = kSplit ? G / 2 : G;
-        const int hl = gl & (H - 1);
         const float Ax = fmaf(2.0f, alx, -EM_), Ay = fmaf(2.0f, aly, -EM_), Az = fmaf(2.0f, alz, -EM_);
         const float Bx = fmaf(2.0f, ahx, EM_), By = fmaf(2.0f, ahy, EM_), Bz = fmaf(2.0f, ahz, EM_);
         const float dw4 = 4.0f * dwmax;
         bool cut = false;
 #pragma unroll
-        for (int k = 0; k < V / H; ++k) {
-            const int v = hl + H * k;
-            if (!((valid[(H * k) >> 6] >> (((H * k) & 63) + hl)) & 1ull)) continue;
-            const float4 p = S->vpos[v];
+        for (int k = 0; k < kRows; ++k) {
+            if (!own(valid, k)) continue;
+            const float4 p = S->vpos[gl + G * k];
             const float rx = fabsf(p.x) + p.w, ry = fabsf(p.y) + p.w, rz = fabsf(p.z) + p.w;
             const float r2 = fmaf(rx, rx, fmaf(ry, ry, rz * rz)) * (1.0f + 4.0f * kSlack);
             // distance to the box per axis: y minus y clamped to [A, B]
@@ -654,8 +634,7 @@ struct Group {
             const float d2 = fmaf(tx, tx, fmaf(ty, ty, tz * tz));
             cut |= !(d2 * (1.0f - kSlack) > r2 + dw4);
         }
-        const uint64_t lanes = (H == 64 ? ~0ull : ((1ull << H) - 1ull)) << (gshift + (gl & ~(H - 1)));
-        return (__ballot(cut) & lanes) == 0ull;
+        return !gany(cut);
     }
 
     // ---------------------------------------------------------- planes
@@ -800,7 +779,7 @@ struct Group {
             tr = has_tri ? S->tmp[gl] : 0u;
             const uint32_t t0 = tri_get<kB>(tr, 0), t1 = tri_get<kB>(tr, 1), t2 = tri_get<kB>(tr, 2);
             bool tw0 = false, tw1 = false, tw2 = false;
-            if constexpr (G == 64 && P <= 256) {
+            if constexpr (P <= 256) {
                 // The dual of a cell is a triangulated sphere: a pair of
                 // planes lies in at most two triangles, which then share it
                 // as an edge.  So the twin of edge (x, y) is removed iff
@@ -1159,7 +1138,7 @@ struct Group {
                     ref = __float_as_uint(hi.w);
                     if (binary) ref = gl < 2 ? (is_leaf(ref) ? ref : ref | kWideBinary) : kWideNone;
                     const bool need = gl < 16 && ((left >> (gl & 15)) & 1u) != 0u && ref != kWideNone &&
-                                      !node_prunable<false, kOctants>(lo, hi, key);
+                                      !node_prunable<kOctants>(lo, hi, key);
                     left = (uint32_t)__ballot(need);
                     key = need ? key : FLT_MAX;
                     fresh = true;
@@ -1174,7 +1153,7 @@ struct Group {
                     const float4 clo = make_float4(rl(lo.x, c), rl(lo.y, c), rl(lo.z, c), rl(lo.w, c));
                     const float4 chi = make_float4(rl(hi.x, c), rl(hi.y, c), rl(hi.z, c), 0.0f);
                     float unused;
-                    found = !node_prunable<false, kBalls>(clo, chi, unused);
+                    found = !node_prunable<kBalls>(clo, chi, unused);
                     r = rl(ref, c);
                 }
             }
@@ -1323,17 +1302,6 @@ struct Group {
         in_guess = false;
     }
 
-    // The owners of the planes held, in plane order (point ids in the index's
-    // order, negative for the box planes, -1 past them), for the large tier
-    // (group op).
-    __device__ __forceinline__ void store_owners(int32_t *out) const {
-#pragma unroll
-        for (int k = 0; k < kPRows; ++k) {
-            const int p = gl + G * k;
-            if (p < kPromoPlanes) out[p] = p < np ? __float_as_int(S->plx[p].y) : -1;
-        }
-    }
-
     // Offers the planes a smaller tier held when it gave the cell up (point
     // ids, negative for none): the cell starts from nearly all of its faces.  They
     // join the Bloom mask, and every later candidate that hits the mask is
@@ -1351,13 +1319,11 @@ struct Group {
 
     __device__ __forceinline__ void setup(const CellParams &prm, GroupLDS<V, P> *s, CandLDS<G> *c) {
         const int lane = threadIdx.x & (kWave - 1);
-        const int grp = lane / G;
         S = s;
         C = c;
         stk_node = stk_left = 0u;
         gl = lane & (G - 1);
         lane64 = lane;
-        gshift = grp * G;
         pts = prm.pts;
         perm = prm.perm;
         inv = prm.inv;
@@ -1407,7 +1373,7 @@ __device__ __forceinline__ int batch_find(const int64_t *off, int n_clouds, int6
 }
 
 // ------------------------------------------------------------------ tiers
-constexpr int kT0Lanes = 16, kT0Verts = 64, kT0Planes = 48, kT0Threads = 256;
+constexpr int kT0Lanes = 16, kT0Threads = 256;
 constexpr int kTmLanes = 64, kTmVerts = 192, kTmPlanes = 128, kTmThreads = 128;
 constexpr int kT1Lanes = 64, kT1Verts = 512, kT1Planes = 255, kT1Threads = 128;
 constexpr int kT2Lanes = 64, kT2Verts = 1024, kT2Planes = 1023, kT2Threads = 64;

@@ -666,15 +666,14 @@ struct Tier0 {
         return hit;
     }
 
-    // Offers a batch of up to G candidates (lane-specific j when `has`);
-    // returns whether the cell changed.
-    __device__ __forceinline__ bool offer_batch(bool has, uint32_t j) {
+    // Offers a batch of up to G candidates (lane-specific j when `has`).
+    __device__ __forceinline__ void offer_batch(bool has, uint32_t j) {
         float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
         bool emptied = false, maybe_guess = true;
         bool live_c = has && prepare(j, c, emptied, maybe_guess);
         if (gany(emptied)) {
             empty_cell();
-            return true;
+            return;
         }
         uint32_t todo = gballot(live_c);
         const uint32_t skipped = gballot(has) & ~todo;
@@ -682,7 +681,7 @@ struct Tier0 {
             if (skipped) count(kStatSkipped, (uint32_t)__popc(skipped));
             if (todo) count(kStatCandidates, (uint32_t)__popc(todo));
         }
-        if (!todo) return false;
+        if (!todo) return;
         // Every vertex against the lane's own candidate: one that lies
         // certainly behind all of them does not cut (the cell only shrinks
         // after this), so only the others are offered one at a time.
@@ -691,7 +690,7 @@ struct Tier0 {
             const bool cuts = may_cut(c);  // (by all lanes of the group)
             live_c = live_c && cuts;
             todo = gballot(live_c);
-            if (!todo) return false;
+            if (!todo) return;
         }
         // the owner's sign bit marks a candidate that may already own a plane
         if (live_c) {
@@ -714,16 +713,16 @@ struct Tier0 {
             if (ow < 0 && bloom && has_plane(owner)) continue;
             if (clip(q, owner)) {
                 if (gl == 0) count(kStatClips);
-                if (status != kSuccess) return true;
+                if (status != kSuccess) return;
             } else if (overflow) {
-                return true;
+                return;
             }
         }
         lds_fence();  // (the next batch is staged in the same place)
-        if (!dirty) return false;
-        update_bounds();
-        dirty = false;
-        return true;
+        if (dirty) {
+            update_bounds();
+            dirty = false;
+        }
     }
 
     // Box plane `code` (2 axis + side) of the cell of seed point sp.  (A
