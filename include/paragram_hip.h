@@ -48,7 +48,8 @@ extern "C" {
  * 17..23 original ids (plus 1) of the first cells with such a test,
  * 24 cells the FP32-only tier gave up on at a removal test its filter could
  * not decide, 25 ... at a new vertex of uncertain orientation (those cells
- * are rebuilt by the FP64-capable twin), 26..31 reserved. */
+ * are rebuilt by tier m), 26..31 the removal tests taken by their FP32 sign
+ * (see pg_compute_cells). */
 #define PG_NUM_STATS 32
 
 /* ABI version compiled into the library (== PG_ABI_VERSION). */
@@ -65,7 +66,10 @@ int pg_index_workspace_bytes(int64_t n, uint64_t *bytes);
 
 /* Builds the LBVH over points (n x 3 float32, optional weights n float32):
  * exact AABB and FP32 clipping box, Morton sort, Karras hierarchy, AABB and
- * max-weight refit.  leaf_size < 0 selects the default.
+ * max-weight refit, and its 16-wide form with leaves of up to 32 points, which
+ * the cells walk.  leaf_size (< 0: the default, 32): points per leaf of the
+ * LBVH, which pg_knn and the guesses of more than 196608 points walk; it
+ * changes their speed, never a result.
  * Replaces pack_points_kernel / combine_points_weights_kernel
  * (voronoi_ultra.cu:30-37, laguerre_ultra.cu:31-41), build_cubql_bvh_and_knn
  * and build_pwr_bvh_and_knn (pwr_bvh.cu:217-339) and the root-box read of
@@ -133,7 +137,7 @@ int pg_row_pool_elems(int64_t cells, uint64_t *elems);
  * stats: PG_NUM_STATS counters, accumulated (stats[26]: removal tests tier 0
  * took by their FP32 sign, all decided in FP64 after it; stats[27]: those
  * whose sign was wrong (or whose vertex lay on a plane of a predicted cube),
- * their cells rebuilt by the FP64-capable instance;
+ * their cells rebuilt by tier m;
  * stats[28..31]: original ids + 1 of the first such cells).
  * cell_cycles: optional (may be null) per-cell cost in GPU clock cycles,
  * original order; bit 31 set marks cells built by a large-capacity tier.

@@ -1,5 +1,6 @@
 // Cell construction for gfx950: shared definitions and the launcher.  The
-// kernels (capacity tiers 0 and 1) are in pg_group_cell.hpp.
+// kernels are in pg_tier0_cell.hpp (tier 0, FP32 only) and pg_group_cell.hpp
+// (tiers m, 1 and 2, with FP64 and exact arithmetic).
 //
 // Replaces compute_bvh_voronoi_kernel (voronoi_ultra.cu:39-141) and
 // compute_bvh_power_diagram_kernel (laguerre_ultra.cu:43-174) together with
@@ -65,7 +66,7 @@ struct CellParams {
     unsigned long long *stats;
     uint32_t *counters;           // [0] tier-0 work, [1] tier-m queue length, [2] tier-m work,
                                   // [3] tier-2 queue length, [4] tier-2 work,
-                                  // [5] cells flagged for FP64 tier 0, [6] FP64 tier-0 windows,
+                                  // [5] cells flagged for tier m, [6] unused,
                                   // [7] removal tests recorded by tier 0 (taken by their FP32 sign),
                                   // [8] tier-1 queue length, [9] tier-1 work
     unsigned long long *pool_top; // row-pool allocation counter (in the scratch, zeroed per launch)
@@ -73,7 +74,7 @@ struct CellParams {
     uint32_t *big_list;           // tier-1 queue of sorted cell ids (room for every cell)
     uint32_t *huge_list;          // tier-2 queue of sorted cell ids (room for every cell)
     uint32_t queue_cap;           // end - begin
-    uint32_t *exact_list;         // [end - begin] flags: cell for the FP64 tier-0 instance
+    uint32_t *exact_list;         // [end - begin] flags: cell that tier m has to rebuild
     int32_t *promo;               // [promo_cap][kPromoPlanes] plane owners of the cells queued for tier m
     uint32_t promo_cap;           // queue slots that keep their owners
     uint32_t *tent;               // [tent_cap][5] tests tier 0 took by their FP32 sign: sorted cell id (or
@@ -170,8 +171,8 @@ __global__ void cell_prep_kernel(uint32_t *counters) {
 }
 
 // Every tier keeps its cells in LDS: the scratch holds the work counters,
-// the row-pool counter, four per-cell lists (the FP64 tier-0 flags and the
-// tier-m, tier-1 and tier-2 queues, each with room for every cell, so no
+// the row-pool counter, four per-cell lists (the flags of cells for tier m
+// and the tier-m, tier-1 and tier-2 queues, each with room for every cell, so no
 // queue can fill), the plane owners of the first cells queued for tier m
 // (room for one cell in 32, and 64 more; a cell past them starts without) and
 // the removal tests tier 0 took by their FP32 sign (room for one test per two

@@ -1422,11 +1422,13 @@ __device__ __forceinline__ uint64_t pool_take(const CellParams &P, uint32_t n) {
 }
 
 // Queues the cells flagged by tier 0 and by the check of its recorded tests
-// for tier m, with no plane owners.  (An FP64 twin of tier 0, 16 lanes per
-// cell, rebuilt them before when more than 2048 were flagged; a wave per cell
-// is the faster of the two at every count: 500 k points with a predicted cube
+// for tier m, with no plane owners.  (An FP64 form of tier 0, 16 lanes per
+// cell, rebuilt them before when more than 2048 were flagged.  A wave per cell
+// is the faster of the two nearly everywhere: 500 k points with a predicted cube
 // 13.3 -> 12.1 ms, 100 k 5.3 -> 3.5, 2 M 50.7 -> 48.4, 640 k flagged cells of 256
-// LiDAR clouds 587 -> 571.)
+// LiDAR clouds 587 -> 571, 61 k points on a 64^3 grid 76.9 -> 42.9, a 20^3 lattice
+// 97.1 -> 16.3.  It is the slower one with a predicted cube on 10 M points, 209 ->
+// 218 ms, of which tier m takes 20.9.)
 __global__ void __launch_bounds__(256) cell_flagged_kernel(const CellParams prm) {
     if (prm.counters[5] == 0u) return;  // no cell was flagged
     const int64_t count = prm.end - prm.begin;

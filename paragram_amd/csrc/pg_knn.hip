@@ -180,9 +180,13 @@ constexpr int kGroupStack = 32;
 // lane per query does less work in total but is a serial chain of some 300
 // dependent loads, as long as the longest query of its wave, and few waves
 // are in flight.  Whole calls with groups / with lanes: uniform points 1 k
-// 0.55 / 0.74 ms, 16 k 0.93 / 1.10, 100 k 2.72 / 2.78, 200 k 4.65 / 4.65,
-// 350 k 7.51 / 7.43, 1 M 19.0 / 18.4; clustered points (x^4) 100 k 3.25 /
-// 4.13, 200 k 5.66 / 6.76 ms.
+// 0.55 / 0.74 ms, 16 k 0.93 / 1.10, 50 k 1.82 / 1.98, 100 k 2.65 / 2.73,
+// 197 k 4.38 / 4.39, 350 k 7.18 / 7.14, 1.4 M 25.9 / 24.8; 90% in 64 clusters
+// 50 k 2.06 / 2.39, 197 k 4.62 / 4.70, 350 k 7.60 / 7.53, 1.4 M 33.9 / 32.7; half
+// in 256 clusters 197 k 4.58 / 4.68, 350 k 7.38 / 7.47, 700 k 13.4 / 13.2; LiDAR
+// scans 50 k 7.26 / 7.48, 197 k 16.6 / 16.7, 350 k 20.9 / 20.8, 700 k 45.6 / 45.1.
+// Only strongly graded points (x^4 of uniform ones) favour groups at every
+// size: 197 k 5.2 / 6.5, 350 k 9.1 / 10.7, 1.4 M 38.4 / 40.9.
 constexpr int64_t kGroupQueries = 3 << 16;
 
 // One compare-exchange of a sorting network over a row: the lane and its

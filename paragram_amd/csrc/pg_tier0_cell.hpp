@@ -27,18 +27,23 @@
 // boundary edges of a clip and the new vertices they make, bounds reductions
 // and the row sort.  All control decisions are group-uniform.
 //
-// The kernel is bound by VALU issue (rocprofv3: 93% of the cycles), not by
-// memory or latency, so a step is worth what it saves in instructions.
+// The kernel is bound by VALU issue (rocprofv3, 1 M uniform points: 7.89e9
+// wave instructions fill 89% of the issue slots, with 38 of 64 lanes active), not
+// by memory or latency, so a step is worth what it saves in instructions.
 // Against four cells that share a binary walk (32 vertex slots with a valid
 // mask, both children of a node tested by every lane), one group walking the
 // 16-wide form for itself visits a tenth of the nodes, and its lanes test
 // different boxes: 8.1e9 instructions in place of 10.2e9 on 1 M uniform
-// points, and the tier took 15.7 ms in place of 20.2 (14.6 with the later steps).  The exact ball test
-// of a child is put off until the walk comes to it, and is done by the whole
-// group, a vertex per lane: testing it for each child by that child's lane
-// took 23.7 ms.  The walk itself is written as selects in one loop that the
-// wave steps through together (20.9 -> 20.0 ms): in divergent branches each
-// join copies the walk's state.
+// points, and the tier took 15.7 ms in place of 20.2 (14.5 with the later
+// steps).  The exact ball test of a child is put off until the walk comes to
+// it, and is done by the whole group, a vertex per lane: testing it for each
+// child by that child's lane took 23.7 ms.  The walk itself is written as
+// selects in one loop that the wave steps through together (20.9 -> 20.0 ms):
+// in divergent branches each join copies the walk's state.
+//
+// The lanes of a group exchange planes, vertices, lists and candidates through
+// LDS; each exchange goes across lds_fence(), which costs nothing measurable
+// (1 M uniform 17.28 -> 17.30 ms, 256 LiDAR clouds 572.8 -> 572.8).
 #pragma once
 
 namespace pg {
@@ -800,9 +805,10 @@ struct Tier0 {
     // the points of the hierarchy that may cut it.
     //
     // Each cell walks the 16-wide hierarchy on its own, depth first, one lane
-    // per child: a node's children are tested once on arrival (and again,
-    // those left, after the cell has changed or when the walk comes back),
-    // then taken by the smallest lower bound of H.  The groups of a wave step
+    // per child: a node's children are tested against the cell's box on arrival
+    // (and again, those left, when the walk comes back from below), then taken
+    // by the smallest lower bound of H, each after a test against the vertices
+    // that the cell has by then.  The groups of a wave step
     // until each has a leaf to offer or has ended, and offer their batches
     // together, so the candidates and clips of the four cells share their
     // instructions.  The reference pops the smallest key from a list instead
